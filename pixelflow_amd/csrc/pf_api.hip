@@ -66,6 +66,16 @@ struct pf_ctx {
     uint8_t *UNIT32 = nullptr;      // mixed precision: the same flags of the FP32 porosity
     bool unit_half = false;         // unit waves hold half the cells or more: the residual and
                                     // the multigrid's level-0 kernels use the flags too
+    // solves of a fixed count in one launch with the grid resident on chip (pf_resident.hip):
+    // the tiling, the waves' unit bits and coefficient sets and the tiles' message buffers
+    bool resident = false;
+    pf::ResidentPlan rpl{};
+    void *rcoef = nullptr;          // double or float by precision, sized by the porosity
+    size_t rcoef_cap = 0;
+    uint32_t *rmask = nullptr, *rfirst = nullptr;
+    unsigned long long *rinbox = nullptr;
+    uint32_t rseq = 1;              // next unused message sequence number
+    unsigned long long *rfail = nullptr;   // set by a launch whose bounded wait ran out
     int err_cap = 0, nparts = 0;
     bool have_phi = false, have_init = false;
     bool timing = false;
@@ -134,6 +144,24 @@ static bool unit_wanted(const pf_desc *d) {
     return !(u && *u && std::atoi(u) == 0);
 }
 
+// Solves of a fixed SOR count run resident on chip where the grid fits (pf_resident.hip),
+// unless the environment selects a variant of the per-half-sweep kernels.
+static bool resident_wanted(const PfGeom &g, const pf_desc *d, pf::ResidentPlan &pl) {
+    if (g.dim != 3 || (d->residual_tol > 0 && d->solver == PF_SOLVER_MG)) return false;
+    const char *own = std::getenv("PF_RESIDENT");
+    if (!(own && *own))
+        for (const char *v : {"PF_SOR_VARIANT", "PF_SWEEP_KB", "PF_SWEEP_XW", "PF_XCD_REMAP", "PF_UNIT_PHI",
+                              "PF_PHI_CODE", "PF_FUSED"}) {
+            const char *e = std::getenv(v);
+            if (e && *e) return false;
+        }
+    return pf::resident_plan(g, d->precision == PF_PREC_MIXED ? 4 : 8, pf::RESIDENT_CUS, pl);
+}
+static int64_t resident_bytes(const pf_desc *d, const pf::ResidentPlan &pl) {
+    const int elem = d->precision == PF_PREC_MIXED ? 4 : 8;
+    return (int64_t)pf::resident_waves(pl) * 8 + pf::resident_inbox_words(pl, elem) * 8;
+}
+
 extern "C" int64_t pf_footprint_bytes(const pf_desc *d) {
     std::string why;
     if (!desc_ok(d, why)) return -1;
@@ -153,7 +181,9 @@ extern "C" int64_t pf_footprint_bytes(const pf_desc *d) {
     tb2_params(g, d, tk, tr);
     const int64_t p2 = (tk > 0) ? (int64_t)8 * 2 * g.HS : 0;
     const int64_t unit = unit_wanted(d) ? unit_flags_size(g) * (d->precision == PF_PREC_MIXED ? 2 : 1) : 0;
-    return (int64_t)8 * (nat * g.NS + spl * 2 * g.HS + interior) + mixed + mg + coded + p2 + unit + 4096;
+    pf::ResidentPlan pl;
+    const int64_t res = resident_wanted(g, d, pl) ? resident_bytes(d, pl) : 0;
+    return (int64_t)8 * (nat * g.NS + spl * 2 * g.HS + interior) + mixed + mg + coded + p2 + unit + res + 4096;
 }
 
 static int alloc(pf_ctx *c, double **p, int64_t n) {
@@ -182,6 +212,10 @@ static void release(pf_ctx *c) {
     if (c->PHTAB) { (void)hipFree(c->PHTAB); c->PHTAB = nullptr; }
     if (c->UNIT) { (void)hipFree(c->UNIT); c->UNIT = nullptr; }
     if (c->UNIT32) { (void)hipFree(c->UNIT32); c->UNIT32 = nullptr; }
+    if (c->rcoef) { (void)hipFree(c->rcoef); c->rcoef = nullptr; }
+    if (c->rmask) { (void)hipFree(c->rmask); c->rmask = nullptr; }
+    if (c->rfirst) { (void)hipFree(c->rfirst); c->rfirst = nullptr; }
+    if (c->rinbox) { (void)hipFree(c->rinbox); c->rinbox = nullptr; }
     if (c->mg32) { pf::mg_destroy(*c->mg32); delete c->mg32; c->mg32 = nullptr; }
     if (c->mg64) { pf::mg_destroy(*c->mg64); delete c->mg64; c->mg64 = nullptr; }
     for (hipEvent_t e : c->evs) (void)hipEventDestroy(e);
@@ -229,6 +263,25 @@ extern "C" int pf_create(const pf_desc *desc, pf_ctx **out) {
         }
     }
     c->nparts = pf::sor_blocks(g);
+    {
+        int cus = 0, coop = 0;
+        c->resident = resident_wanted(g, desc, c->rpl) &&
+                      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess &&
+                      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess &&
+                      coop && c->rpl.bx * c->rpl.by * c->rpl.bz <= cus;
+    }
+    if (c->resident) {
+        const int nw = pf::resident_waves(c->rpl);
+        const int64_t words = pf::resident_inbox_words(c->rpl, desc->precision == PF_PREC_MIXED ? 4 : 8);
+        c->nparts = std::max(c->nparts, nw);
+        if (hipMalloc((void **)&c->rmask, (size_t)nw * 4) != hipSuccess ||
+            hipMalloc((void **)&c->rfirst, (size_t)nw * 4) != hipSuccess ||
+            hipMalloc((void **)&c->rinbox, (size_t)words * 8) != hipSuccess) {
+            rc = fail(c, PF_ENOMEM, "hipMalloc of the resident sweep's arrays failed");
+            goto bad;
+        }
+        pf::launch_clear_u64(c->st, c->rinbox, (int)words);
+    }
     if (hipMalloc((void **)&c->err_part, sizeof(unsigned long long) * (size_t)c->nparts) != hipSuccess ||
         hipMalloc((void **)&c->res_part, sizeof(unsigned long long) * (size_t)c->nparts) != hipSuccess ||
         hipMalloc((void **)&c->res_val, sizeof(unsigned long long)) != hipSuccess) {
@@ -378,6 +431,36 @@ extern "C" int pf_sync(pf_ctx *c) {
 // ------------------------------------------------------------------------------------
 // Porosity: grid_conditions* (src/omp_parallel/lib/grid.f90) on the host, once.
 // ------------------------------------------------------------------------------------
+// The resident sweep's masks and coefficient sets.  Without room for the sets the
+// per-half-sweep kernels are used.
+static int resident_from_porosity(pf_ctx *c) {
+    const bool f32 = c->d.precision == PF_PREC_MIXED, fast = c->sor_variant == 2;
+    auto setup = [&](const uint32_t *first) {
+        if (f32) pf::launch_resident_setup<float>(c->st, c->g, c->a, c->rpl, c->PHI32, c->phi, (float *)c->rcoef, c->rmask, first, fast);
+        else pf::launch_resident_setup<double>(c->st, c->g, c->a, c->rpl, c->PHIs, c->phi, (double *)c->rcoef, c->rmask, first, fast);
+    };
+    std::vector<uint32_t> mask((size_t)pf::resident_waves(c->rpl)), first;
+    setup(nullptr);
+    PF_TRY_HIP(c, hipMemcpyAsync(mask.data(), c->rmask, mask.size() * 4, hipMemcpyDeviceToHost, c->st));
+    PF_TRY_HIP(c, hipStreamSynchronize(c->st));
+    const size_t bytes = (size_t)std::max<int64_t>(1, pf::resident_sets(c->rpl, mask, first)) * pf::RESIDENT_SET * (f32 ? 4 : 8);
+    if (bytes > c->rcoef_cap) {
+        if (c->rcoef) (void)hipFree(c->rcoef);
+        c->rcoef = nullptr;
+        c->rcoef_cap = 0;
+        if (hipMalloc(&c->rcoef, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            c->rcoef = nullptr;
+            return PF_OK;
+        }
+        c->rcoef_cap = bytes;
+    }
+    PF_TRY_HIP(c, hipMemcpyAsync(c->rfirst, first.data(), first.size() * 4, hipMemcpyHostToDevice, c->st));
+    setup(c->rfirst);
+    PF_TRY_HIP(c, hipStreamSynchronize(c->st));   // `first` is on this stack frame
+    return PF_OK;
+}
+
 // Time-invariant data derived from porosity: stored faces, the colour-split porosity and
 // the choice of sweep kernel.
 static int derive_from_porosity(pf_ctx *c) {
@@ -397,6 +480,10 @@ static int derive_from_porosity(pf_ctx *c) {
     PF_TRY_HIP(c, hipGetLastError());
     c->sor_variant = (hbad == 0) ? 2 : 1;
     if (c->sor_forced >= 0 && c->sor_forced <= 2 && !(c->sor_forced == 2 && hbad != 0)) c->sor_variant = c->sor_forced;
+    if (c->resident) {
+        const int rc = resident_from_porosity(c);
+        if (rc != PF_OK) return rc;
+    }
     c->unit_cells = 0;
     if (c->UNIT) {
         pf::launch_unit_flags(c->st, g, c->PHIs, c->UNIT);
@@ -545,6 +632,29 @@ extern "C" int pf_initial(pf_ctx *c) {
 // ------------------------------------------------------------------------------------
 // The time step
 // ------------------------------------------------------------------------------------
+// A solve of `iters` iterations as one resident launch; false where it does not apply.
+static bool enqueue_resident(pf_ctx *c, unsigned long long *slot, int iters) {
+    // the buffers' reuse needs messages of two iterations; the sequence numbers bound the count
+    if (!c->resident || !c->rcoef || c->fused || c->sor_variant == 0 || iters < 2 || iters >= (1 << 28)) return false;
+    const bool f32 = c->d.precision == PF_PREC_MIXED;
+    if (c->rseq > 0xffffffffu - 2u * (uint32_t)iters) {   // start over on an empty inbox
+        pf::launch_clear_u64(c->st, c->rinbox, (int)pf::resident_inbox_words(c->rpl, f32 ? 4 : 8));
+        c->rseq = 1;
+    }
+    const hipError_t e =
+        f32 ? pf::launch_resident<float>(c->st, c->g, c->a, c->rpl, iters, c->rseq, c->E32, c->R32, (const float *)c->rcoef,
+                                         c->rmask, c->rfirst, c->rinbox, slot, c->rfail)
+            : pf::launch_resident<double>(c->st, c->g, c->a, c->rpl, iters, c->rseq, c->P, c->BB, (const double *)c->rcoef,
+                                          c->rmask, c->rfirst, c->rinbox, slot, c->rfail);
+    if (e != hipSuccess) {   // not launched: the half-sweep kernels take over
+        (void)hipGetLastError();
+        c->resident = false;
+        return false;
+    }
+    c->rseq += 2u * (uint32_t)iters;
+    return true;
+}
+
 static void enqueue_sor(pf_ctx *c, unsigned long long *slot, int iters) {
     const PfGeom &g = c->g;
     const bool periodic = (c->d.bc == PF_BC_UNIFORM);
@@ -555,6 +665,7 @@ static void enqueue_sor(pf_ctx *c, unsigned long long *slot, int iters) {
     // 3D sweeps (i+j+k) even first (:493), 2D sweeps (i+j) odd first (:339)
     const int first = (g.dim == 3) ? 0 : 1;
     int done = 0;
+    if (enqueue_resident(c, slot, iters)) return;
     if (c->tb2_k > 0 && c->sor_variant != 0 && iters >= 2) {
         // K iterations per launch, P -> P2 -> P ...: an even number of launches leaves the
         // result in P, so a launch of two or more iterations is split when the count is odd
@@ -665,7 +776,7 @@ static int enqueue_mixed(pf_ctx *c, unsigned long long *slot, double *res, int *
             if ((rc = residual(false)) != PF_OK) return rc;
         }
         const int kk = tol_mode ? K : (remaining < K ? remaining : K);
-        int done = 0;
+        int done = enqueue_resident(c, slot, kk) ? kk : 0;
         if (c->fused && kk >= 2) {
             // E2's non-periodic ghosts are 0 like E's (zeroed at allocation, never written)
             for (; done + 2 <= kk; done += 2) {
@@ -756,10 +867,11 @@ extern "C" int pf_step(pf_ctx *c, int nsteps, pf_stats *stats) {
     if (c->err_cap < nsteps) {
         if (c->err) PF_TRY_HIP(c, hipFree(c->err));
         c->err = nullptr;
-        PF_TRY_HIP(c, hipMalloc((void **)&c->err, sizeof(unsigned long long) * (size_t)nsteps));
+        PF_TRY_HIP(c, hipMalloc((void **)&c->err, sizeof(unsigned long long) * ((size_t)nsteps + 1)));
         c->err_cap = nsteps;
     }
-    pf::launch_clear_u64(c->st, c->err, nsteps);
+    pf::launch_clear_u64(c->st, c->err, nsteps + 1);
+    c->rfail = c->err + nsteps;
     c->mixed_res.clear();
     c->mixed_cycles.clear();
     c->mixed_iters.clear();
@@ -806,9 +918,11 @@ extern "C" int pf_step(pf_ctx *c, int nsteps, pf_stats *stats) {
         pf::launch_boundary(c->st, g, c->a, c->phi, c->u, c->v, c->w, c->P);
         PF_TRY_HIP(c, hipGetLastError());
     }
-    std::vector<unsigned long long> e((size_t)nsteps);
-    PF_TRY_HIP(c, hipMemcpyAsync(e.data(), c->err, sizeof(unsigned long long) * (size_t)nsteps, hipMemcpyDeviceToHost, c->st));
+    std::vector<unsigned long long> e((size_t)nsteps + 1);
+    PF_TRY_HIP(c, hipMemcpyAsync(e.data(), c->err, sizeof(unsigned long long) * e.size(), hipMemcpyDeviceToHost, c->st));
     PF_TRY_HIP(c, hipStreamSynchronize(c->st));
+    if (e[(size_t)nsteps] != 0)
+        return fail(c, PF_EHIP, "resident sweep: a tile's wait for its neighbours ran out (PF_RESIDENT=0 avoids it)");
     if (c->timing && c->d.iter_max > 0) {
         double sweep_ms = 0.0;
         for (int s = 0; s < nsteps; ++s) {

@@ -910,14 +910,13 @@ __device__ __forceinline__ double residual_cell(const PfGeom &g, const StepArgs 
     return fabs(r / ap);
 }
 
-// FP32 SOR update of the correction e on A e = r (mixed precision), from the values
-// around the cell; shared by the two-launch and the fused sweep.
+// The six FP32 coefficients of a cell of the correction equation after the boundary rows'
+// rules, and ap (the sum before them).
 template <int DIM>
-__device__ __forceinline__ float sor32_value(const PfGeom &g, const StepArgs &a, int i, int j, int k, float ec,
-                                             float eW, float eE, float eS, float eN, float eB, float eT, float fc,
-                                             float fW, float fE, float fS, float fN, float fB, float fT, float rr,
-                                             const double *__restrict__ phi, float cdx, float cdy, float cdz) {
-    CoefT<float> c;
+__device__ __forceinline__ void sor32_coefs(const PfGeom &g, const StepArgs &a, int i, int j, int k, float fc,
+                                            float fW, float fE, float fS, float fN, float fB, float fT,
+                                            const double *__restrict__ phi, float cdx, float cdy, float cdz,
+                                            CoefT<float> &c, float &ap) {
     c.ae = face32(fE, fc, cdx);
     c.aw = face32(fc, fW, cdx);
     c.an = face32(fN, fc, cdy);
@@ -928,8 +927,20 @@ __device__ __forceinline__ float sor32_value(const PfGeom &g, const StepArgs &a,
         c.at = face32(fT, fc, cdz);
         c.ab = face32(fc, fB, cdz);
     }
-    const float ap = -(c.ae + c.aw + c.an + c.as + c.at + c.ab);
+    ap = -(c.ae + c.aw + c.an + c.as + c.at + c.ab);
     if (is_edge_row(g, a, i, j, k)) row_rules<false, float>(g, a, i, j, k, c, nullptr, nullptr, phi, 0.);
+}
+
+// FP32 SOR update of the correction e on A e = r (mixed precision), from the values
+// around the cell; shared by the two-launch and the fused sweep.
+template <int DIM>
+__device__ __forceinline__ float sor32_value(const PfGeom &g, const StepArgs &a, int i, int j, int k, float ec,
+                                             float eW, float eE, float eS, float eN, float eB, float eT, float fc,
+                                             float fW, float fE, float fS, float fN, float fB, float fT, float rr,
+                                             const double *__restrict__ phi, float cdx, float cdy, float cdz) {
+    CoefT<float> c;
+    float ap;
+    sor32_coefs<DIM>(g, a, i, j, k, fc, fW, fE, fS, fN, fB, fT, phi, cdx, cdy, cdz, c, ap);
     float num = rr - c.ae * eE - c.aw * eW - c.an * eN - c.as * eS;
     if (DIM == 3) num = num - c.at * eT - c.ab * eB;
     const float om = (float)a.omega;

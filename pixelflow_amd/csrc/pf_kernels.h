@@ -108,6 +108,34 @@ void launch_sor_fused(hipStream_t st, const PfGeom &g, const StepArgs &a, const 
                       bool fast);
 void launch_sor32_fused(hipStream_t st, const PfGeom &g, const StepArgs &a, const float *A, float *B, const float *F,
                         const float *R, const double *phi, unsigned long long *slot, int track);
+// Colour sweeps of a whole solve in one launch, the grid resident on chip (pf_resident.hip).
+// bx, by, bz: tiles per axis; tx, ty, tz: cells of a tile; ns: height pairs per thread;
+// threads: per block.
+struct ResidentPlan {
+    int bx, by, bz, tx, ty, tz, ns, threads;
+};
+constexpr int RESIDENT_CUS = 256;   // compute units of an MI355X: one workgroup on each
+// The tiling for one workgroup per CU on `cus` CUs, for elements of `elem` bytes; false
+// where the grid does not fit.  PF_RESIDENT="bx,by,bz" in the environment sets the tiles per
+// axis ("0": never).
+bool resident_plan(const PfGeom &g, int elem, int cus, ResidentPlan &pl);
+int64_t resident_inbox_words(const ResidentPlan &pl, int elem);
+// Waves of a launch, one error slot and one entry of `mask` and `first` each.
+int resident_waves(const ResidentPlan &pl);
+// From the waves' masks: each wave's first coefficient set, and their count; a set is
+// RESIDENT_SET elements.
+constexpr int RESIDENT_SET = 7 * 64;
+int64_t resident_sets(const ResidentPlan &pl, const std::vector<uint32_t> &mask, std::vector<uint32_t> &first);
+// Without `first` writes the masks, with it the coefficient sets (in pf_resident.hip).
+template <typename T>
+void launch_resident_setup(hipStream_t st, const PfGeom &g, const StepArgs &a, const ResidentPlan &pl, const T *PHI,
+                           const double *phi, T *coef, uint32_t *mask, const uint32_t *first, bool fast);
+// iters red/black iterations, even cells first, on X (colour-split, ghosts current) with right-hand side R.
+// Half-sweep h's messages carry seq + h, which no earlier launch on this inbox may have used.
+template <typename T>
+hipError_t launch_resident(hipStream_t st, const PfGeom &g, const StepArgs &a, const ResidentPlan &pl, int iters,
+                           uint32_t seq, T *X, const T *R, const T *coef, const uint32_t *mask, const uint32_t *first_set,
+                           unsigned long long *inbox, unsigned long long *slots, unsigned long long *fail);
 // Body force (pressure + wall-force terms): partial holds force_blocks(g)*6 doubles, out 6.
 int force_blocks(const PfGeom &g);
 void launch_force(hipStream_t st, const PfGeom &g, const StepArgs &a, const double *phi, const double *u,

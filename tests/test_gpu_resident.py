@@ -1,0 +1,76 @@
+"""Solves run as one launch with the grid resident on chip (pf_resident.hip).
+
+FP64 against the oracle bit for bit, the FP32 correction sweeps against the per-half-sweep
+kernels bit for bit (the same operations on the same operands), over tilings with one and
+many tiles per axis, ragged last tiles, one to sixteen height pairs per thread, even and odd
+periodic extents (an odd one wraps a colour onto itself) and the rooms' walls.
+"""
+import numpy as np
+import pytest
+
+from pixelflow_amd import cases
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(bc, size, iters, steps):
+    m, n, l = size
+    if bc == "air":
+        return cases.room_case(5, steps=steps, iter_max=iters, size=size)
+    dx = 0.01
+    p = cases.CaseParams(dim=3, m=m, n=n, l=l, width=dx * (m - 1), height=dx * (n - 1), depth=dx * (l - 1),
+                         time=1e-4 * steps, istep_max=steps, iter_max=iters)
+    rng = np.random.default_rng(m * n + l)
+    phi = np.ones((l, n, m))
+    some = rng.random(phi.shape) < 0.01          # isolated cells, so unit and other waves both occur
+    phi[some] = rng.uniform(0.0, 1.0, int(some.sum()))
+    phi[l // 3:l // 2, n // 3:n // 2, m // 3:m // 2] = rng.uniform(0.0, 1.0)
+    return p, phi
+
+
+RUNS = [
+    ("uniform", (64, 32, 32), "2,1,2", 7),       # 32x32 tiles, eight height pairs
+    ("uniform", (64, 32, 32), "4,2,8", 6),
+    ("uniform", (33, 27, 19), "2,2,3", 5),       # odd periodic extents, ragged tiles
+    ("uniform", (45, 28, 9), "2,1,9", 4),        # one-cell-thick tiles, a tile its own neighbour in y
+    ("uniform", (30, 32, 7), "1,1,1", 3),        # a single tile, its own neighbour in y and z
+    ("uniform", (41, 21, 16), "3,4,2", 2),       # the fewest iterations of a resident solve
+    ("uniform", (97, 65, 49), "", 9),            # the rule's own tiling
+    ("air", (64, 48, 40), "2,2,3", 6),
+    ("air", (48, 40, 33), "", 5),
+]
+
+
+@pytest.mark.parametrize("bc,size,tiles,iters", RUNS)
+def test_resident_solve_matches_oracle(bc, size, tiles, iters, monkeypatch):
+    import pyoracle
+    from pixelflow_amd.solver import Solver
+    if tiles:
+        monkeypatch.setenv("PF_RESIDENT", tiles)
+    print(f"[gpu] resident {bc} {size} tiles={tiles or 'rule'} iters={iters}", flush=True)
+    p, phi = _case(bc, size, iters, 3)
+    o = pyoracle.OracleRun(p, phi)
+    ref = o.step(3)
+    with Solver(p, phi) as s:
+        st = s.step(3)
+        for f in ("u", "v", "w", "p"):
+            np.testing.assert_array_equal(s.interior(f), o.interior(f), err_msg=f)
+        np.testing.assert_array_equal(st["sor_error"], ref)
+
+
+@pytest.mark.parametrize("bc,size,tiles,iters", RUNS + [("uniform", (64, 64, 64), "2,2,2", 6)])
+def test_resident_fp32_solve_matches_sweeps(bc, size, tiles, iters, monkeypatch):
+    from pixelflow_amd.solver import PF_PREC_MIXED, Solver
+    p, phi = _case(bc, size, iters, 3)
+    out = {}
+    for mode in ("0", tiles):
+        if mode:
+            monkeypatch.setenv("PF_RESIDENT", mode)
+        else:
+            monkeypatch.delenv("PF_RESIDENT")
+        print(f"[gpu] resident FP32 {bc} {size} tiles={mode or 'rule'} iters={iters}", flush=True)
+        with Solver(p, phi, precision=PF_PREC_MIXED, inner_iters=max(2, iters // 2)) as s:
+            st = s.step(3)
+            out[mode == "0"] = [s.interior(f) for f in ("u", "v", "w", "p")] + [st["sor_error"]]
+    for a, b in zip(out[True], out[False]):
+        np.testing.assert_array_equal(a, b)
