@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "../../include/pixelflow.h"
+#include "pf_download.h"
 #include "pf_host.h"
 #include "pf_kernels.h"
 #include "pf_mg.h"
@@ -76,6 +77,7 @@ struct pf_ctx {
     unsigned long long *rinbox = nullptr;
     uint32_t rseq = 1;              // next unused message sequence number
     unsigned long long *rfail = nullptr;   // set by a launch whose bounded wait ran out
+    pf::Downloader down;
     int err_cap = 0, nparts = 0;
     bool have_phi = false, have_init = false;
     bool timing = false;
@@ -220,6 +222,7 @@ static void release(pf_ctx *c) {
     if (c->mg64) { pf::mg_destroy(*c->mg64); delete c->mg64; c->mg64 = nullptr; }
     for (hipEvent_t e : c->evs) (void)hipEventDestroy(e);
     c->evs.clear();
+    c->down.release();
     if (c->st) (void)hipStreamDestroy(c->st);
     c->st = nullptr;
 }
@@ -585,11 +588,7 @@ extern "C" int pf_download(pf_ctx *c, int field, double *host, int64_t ldi, int6
     bool split;
     double *src = field_ptr(c, field, split);
     if (!src) return fail(c, PF_EINVAL, "unknown field");
-    const int64_t size = split ? 2 * g.HS : g.NS;
-    std::vector<double> stage((size_t)size);
-    PF_TRY_HIP(c, hipStreamSynchronize(c->st));
-    PF_TRY_HIP(c, hipMemcpy(stage.data(), src, (size_t)size * sizeof(double), hipMemcpyDeviceToHost));
-    pf::to_host(g, split, stage, host, ldi, ldj);
+    PF_TRY_HIP(c, c->down.get(c->st, g, split, src, host, ldi, ldj));
     return PF_OK;
 }
 

@@ -27,6 +27,7 @@
 
 #include "../../include/pixelflow.h"
 #include "pf_batch.h"
+#include "pf_download.h"
 #include "pf_cells.h"
 #include "pf_device.h"
 #include "pf_host.h"
@@ -350,6 +351,7 @@ __global__ void k_inc_int(int *p) {
 using pf::BatchCase;
 
 struct pf_batch {
+    pf::Downloader down;
     pf_desc kind{};                 // settings shared by every case
     int max_cases = 0;
     hipStream_t st = nullptr;
@@ -566,6 +568,7 @@ extern "C" int pf_batch_destroy(pf_batch *b) {
         if (b->side[q]) (void)hipStreamSynchronize(b->side[q]);
     for (auto &s : b->slots) slot_release_mg(s);
     drop_graphs(b);
+    b->down.release();
     void *ptrs[] = {b->arena, b->d_cases, b->d_nat_prefix, b->d_swp_prefix, b->d_nat_tile, b->d_swp_tile,
                     b->d_face_tile[0], b->d_face_tile[1], b->d_face_tile[2],
                     b->d_active, b->d_step,
@@ -1358,10 +1361,7 @@ extern "C" int pf_batch_download(pf_batch *b, int slot, int field, double *host,
         default: break;
     }
     if (!src) { b->msg = "unknown field"; return PF_EINVAL; }
-    std::vector<double> stage((size_t)(split ? 2 * g.HS : g.NS));
-    PFB_TRY(b, hipStreamSynchronize(b->st));
-    PFB_TRY(b, hipMemcpy(stage.data(), src, stage.size() * 8, hipMemcpyDeviceToHost));
-    pf::to_host(g, split, stage, host, ldi, ldj);
+    PFB_TRY(b, b->down.get(b->st, g, split, src, host, ldi, ldj));
     return PF_OK;
 }
 

@@ -146,16 +146,7 @@ inline void scale_interior(const PfGeom &g, const std::vector<double> &phi, std:
             }
 }
 
-// device layout <-> reference host storage (Fortran order, leading dimensions ldi, ldj)
-inline void to_host(const PfGeom &g, bool split, const std::vector<double> &stage, double *host, int64_t ldi,
-                    int64_t ldj) {
-    for (int k = 0; k < g.Z; ++k)
-        for (int j = 0; j < g.Y; ++j)
-            for (int i = 0; i < g.m + 2; ++i)
-                host[(size_t)i + (size_t)ldi * ((size_t)j + (size_t)ldj * (size_t)k)] =
-                    stage[(size_t)(split ? pf_soff(g, i, j, k) : pf_off(g, i, j, k))];
-}
-
+// reference host storage (Fortran order, leading dimensions ldi, ldj) -> device layout
 inline void from_host(const PfGeom &g, bool split, const double *host, int64_t ldi, int64_t ldj,
                       std::vector<double> &stage) {
     for (int k = 0; k < g.Z; ++k)
