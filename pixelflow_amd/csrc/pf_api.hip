@@ -69,7 +69,7 @@ struct pf_ctx {
                                     // the multigrid's level-0 kernels use the flags too
     // solves of a fixed count in one launch with the grid resident on chip (pf_resident.hip):
     // the tiling, the waves' unit bits and coefficient sets and the tiles' message buffers
-    bool resident = false;
+    bool resident = false, resident2 = false;   // 3D, 2D
     pf::ResidentPlan rpl{};
     void *rcoef = nullptr;          // double or float by precision, sized by the porosity
     size_t rcoef_cap = 0;
@@ -159,6 +159,20 @@ static bool resident_wanted(const PfGeom &g, const pf_desc *d, pf::ResidentPlan 
         }
     return pf::resident_plan(g, d->precision == PF_PREC_MIXED ? 4 : 8, pf::RESIDENT_CUS, pl);
 }
+// The same in 2D (uniform inflow), and the plan for a solve of `iters` iterations.
+static bool resident2_wanted(const PfGeom &g, const pf_desc *d) {
+    pf::Resident2Plan pl;
+    if (g.dim != 2 || (d->residual_tol > 0 && d->solver == PF_SOLVER_MG)) return false;
+    const char *own = std::getenv("PF_RESIDENT");
+    if (!(own && *own))
+        for (const char *v : {"PF_SOR_VARIANT", "PF_SWEEP_XW", "PF_XCD_REMAP", "PF_UNIT_PHI", "PF_PHI_CODE", "PF_FUSED",
+                              "PF_SOR_TB2"}) {
+            const char *e = std::getenv(v);
+            if (e && *e) return false;
+        }
+    const int iters = d->inner_iters > 0 && (d->precision == PF_PREC_MIXED || d->residual_tol > 0) ? d->inner_iters : d->iter_max;
+    return pf::resident2_plan(g, d->bc, std::max(2, iters), pl);
+}
 static int64_t resident_bytes(const pf_desc *d, const pf::ResidentPlan &pl) {
     const int elem = d->precision == PF_PREC_MIXED ? 4 : 8;
     return (int64_t)pf::resident_waves(pl) * 8 + pf::resident_inbox_words(pl, elem) * 8;
@@ -180,11 +194,13 @@ extern "C" int64_t pf_footprint_bytes(const pf_desc *d) {
     const int64_t coded =
         (d->precision == PF_PREC_FP64 && code_on) ? (int64_t)4 * 2 * g.HS + (int64_t)8 * PHI_TAB_MAX : 0;
     int tk = 0, tr = 0;
-    tb2_params(g, d, tk, tr);
+    const bool res2 = resident2_wanted(g, d);
+    if (!res2) tb2_params(g, d, tk, tr);
     const int64_t p2 = (tk > 0) ? (int64_t)8 * 2 * g.HS : 0;
     const int64_t unit = unit_wanted(d) ? unit_flags_size(g) * (d->precision == PF_PREC_MIXED ? 2 : 1) : 0;
     pf::ResidentPlan pl;
-    const int64_t res = resident_wanted(g, d, pl) ? resident_bytes(d, pl) : 0;
+    const int64_t res = resident_wanted(g, d, pl) ? resident_bytes(d, pl)
+                        : res2 ? pf::resident2_inbox_words(g, d->precision == PF_PREC_MIXED ? 4 : 8) * 8 : 0;
     return (int64_t)8 * (nat * g.NS + spl * 2 * g.HS + interior) + mixed + mg + coded + p2 + unit + res + 4096;
 }
 
@@ -272,6 +288,19 @@ extern "C" int pf_create(const pf_desc *desc, pf_ctx **out) {
                       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess &&
                       hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess &&
                       coop && c->rpl.bx * c->rpl.by * c->rpl.bz <= cus;
+        c->resident2 = resident2_wanted(g, desc) &&
+                       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess &&
+                       hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess &&
+                       coop && cus >= pf::RESIDENT_CUS;
+    }
+    if (c->resident2) {
+        const int64_t words = pf::resident2_inbox_words(g, desc->precision == PF_PREC_MIXED ? 4 : 8);
+        c->nparts = std::max(c->nparts, pf::RESIDENT_CUS * 8);
+        if (hipMalloc((void **)&c->rinbox, (size_t)words * 8) != hipSuccess) {
+            rc = fail(c, PF_ENOMEM, "hipMalloc of the resident sweep's arrays failed");
+            goto bad;
+        }
+        pf::launch_clear_u64(c->st, c->rinbox, (int)words);
     }
     if (c->resident) {
         const int nw = pf::resident_waves(c->rpl);
@@ -298,7 +327,7 @@ extern "C" int pf_create(const pf_desc *desc, pf_ctx **out) {
         if (fv && *fv) c->fused = std::atoi(fv) != 0;
         c->fused = c->fused && pf::sor_fused_ok(g, desc->bc);
     }
-    tb2_params(g, desc, c->tb2_k, c->tb2_r);
+    if (!c->resident2) tb2_params(g, desc, c->tb2_k, c->tb2_r);
     if ((c->fused || c->tb2_k > 0) && desc->precision == PF_PREC_FP64 && (rc = alloc(c, &c->P2, 2 * g.HS)) != PF_OK)
         goto bad;
     if (desc->precision == PF_PREC_MIXED) {
@@ -632,7 +661,30 @@ extern "C" int pf_initial(pf_ctx *c) {
 // The time step
 // ------------------------------------------------------------------------------------
 // A solve of `iters` iterations as one resident launch; false where it does not apply.
+static bool enqueue_resident2(pf_ctx *c, unsigned long long *slot, int iters) {
+    pf::Resident2Plan pl;
+    if (!c->resident2 || c->fused || c->sor_variant == 0 || iters >= (1 << 28) ||
+        !pf::resident2_plan(c->g, c->d.bc, iters, pl))
+        return false;
+    const bool f32 = c->d.precision == PF_PREC_MIXED, fast = c->sor_variant == 2;
+    if (c->rseq > 0xffffffffu - (uint32_t)iters) {   // start over on an empty inbox
+        pf::launch_clear_u64(c->st, c->rinbox, (int)pf::resident2_inbox_words(c->g, f32 ? 4 : 8));
+        c->rseq = 1;
+    }
+    const hipError_t e = f32 ? pf::launch_resident2<float>(c->st, c->g, c->a, pl, iters, c->rseq, c->E32, c->R32, c->PHI32,
+                                                           c->phi, fast, c->rinbox, slot, c->rfail)
+                             : pf::launch_resident2<double>(c->st, c->g, c->a, pl, iters, c->rseq, c->P, c->BB, c->PHIs,
+                                                            c->phi, fast, c->rinbox, slot, c->rfail);
+    if (e != hipSuccess) {   // not launched: the half-sweep kernels take over
+        (void)hipGetLastError();
+        c->resident2 = false;
+        return false;
+    }
+    c->rseq += (uint32_t)iters;
+    return true;
+}
 static bool enqueue_resident(pf_ctx *c, unsigned long long *slot, int iters) {
+    if (c->g.dim == 2) return enqueue_resident2(c, slot, iters);
     // the buffers' reuse needs messages of two iterations; the sequence numbers bound the count
     if (!c->resident || !c->rcoef || c->fused || c->sor_variant == 0 || iters < 2 || iters >= (1 << 28)) return false;
     const bool f32 = c->d.precision == PF_PREC_MIXED;

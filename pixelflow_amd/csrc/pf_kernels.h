@@ -136,6 +136,19 @@ template <typename T>
 hipError_t launch_resident(hipStream_t st, const PfGeom &g, const StepArgs &a, const ResidentPlan &pl, int iters,
                            uint32_t seq, T *X, const T *R, const T *coef, const uint32_t *mask, const uint32_t *first_set,
                            unsigned long long *inbox, unsigned long long *slots, unsigned long long *fail);
+// The same in 2D: K iterations between exchanges, R rows a block, `rows` held, q cells of each
+// colour a thread, whole: one block holds the grid.  PF_RESIDENT="K,R" in the environment
+// sets them ("0": never).
+struct Resident2Plan {
+    int K, R, rows, q, blocks, whole;
+};
+bool resident2_plan(const PfGeom &g, int bc, int iters, Resident2Plan &pl);
+int64_t resident2_inbox_words(const PfGeom &g, int elem);
+// Exchange t's messages carry seq + t, at most iters of them.
+template <typename T>
+hipError_t launch_resident2(hipStream_t st, const PfGeom &g, const StepArgs &a, const Resident2Plan &pl, int iters,
+                            uint32_t seq, T *X, const T *R, const T *PHI, const double *phi, bool fast,
+                            unsigned long long *inbox, unsigned long long *slots, unsigned long long *fail);
 // Body force (pressure + wall-force terms): partial holds force_blocks(g)*6 doubles, out 6.
 int force_blocks(const PfGeom &g);
 void launch_force(hipStream_t st, const PfGeom &g, const StepArgs &a, const double *phi, const double *u,

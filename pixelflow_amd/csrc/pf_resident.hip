@@ -696,4 +696,334 @@ template void launch_resident_setup<double>(hipStream_t, const PfGeom &, const S
 template void launch_resident_setup<float>(hipStream_t, const PfGeom &, const StepArgs &, const ResidentPlan &,
                                            const float *, const double *, float *, uint32_t *, const uint32_t *, bool);
 
+// ------------------------------------------------------------------------------------
+// 2D: a block owns R rows over the whole width and holds them with 2K rows on each side.
+// It runs K iterations on its own, every half-sweep updating one row fewer on each side (the
+// rows whose neighbours are still exact), then takes the 2K rows on each side from their
+// owners again: an exchange, which costs as much as several half-sweeps of so few cells, is
+// paid once in K iterations.  A message has four slots, by exchange: where n is no multiple of
+// R, the last block reads one block further than reads it, so a writer may be three exchanges
+// ahead of that reader; such a grid takes three rounds at least, so that its rows are written
+// back in place only after every block has loaded them.  The rows wrap in y.  A grid that one block holds needs no
+// exchange.  p lives in LDS by colour, a cell's right-hand side and coefficients in its
+// thread's registers, Q cells of each colour a thread.
+//
+// With n odd row 1 and row n hold the same colours and each takes the other's value of
+// before the half-sweep (the reference refreshes the ghost rows between half-sweeps): there
+// every thread reads before any writes.  The first half-sweep of a launch takes the ghost
+// rows as they are in memory.
+//
+// Measured, us per iteration, before / resident: 48x24 (one block, q = 2) 3.05 (two iterations
+// a launch) / 0.89; 256x128 4.67 / 2.57 with K,R = 2,1 (q = 3), 2.88 with 1,1 (q = 2), 2.50
+// with 3,1 (q = 4), 2.72 with 2,2; 511x255, odd in y, 16.1 (a launch per half-sweep and per
+// refresh of the ghost rows) / 4.2 with 2,1 (q = 5), 4.6 with 1,1.  A half-sweep is FP64 issue
+// (about 55 instructions a cell) and the latency of one LDS read, update, write and barrier.
+// ------------------------------------------------------------------------------------
+namespace {
+
+constexpr int R2T = 512;      // threads of a block; 256 registers each
+constexpr int R2Q = 5;        // cells of one colour per thread, at most
+
+template <typename T>
+struct Resident2 {
+    PfGeom g;
+    StepArgs a;
+    Resident2Plan pl;
+    int iters;
+    uint32_t seq;      // exchange t carries seq + t
+    T *X;
+    const T *R, *PHI;
+    const double *phi;
+    u64 *inbox;
+    u64 *slots;
+    u64 *fail;
+};
+
+// A cell's coefficients and what its division needs.
+template <typename T>
+struct Cell2;
+template <>
+struct Cell2<double> {
+    double ae, aw, an, as, ap, s, r;
+    template <bool FAST>
+    __device__ __forceinline__ void set(const PfGeom &g, const StepArgs &a, int i, int j, const double *PHI,
+                                        const double *phi) {
+        Coef c;
+        ap = sor_coefs<2, FAST>(g, a, i, j, 0, PHI[pf_soff(g, i, j, 0)], PHI[pf_soff(g, i - 1, j, 0)],
+                                PHI[pf_soff(g, i + 1, j, 0)], PHI[pf_soff(g, i, j - 1, 0)], PHI[pf_soff(g, i, j + 1, 0)],
+                                0., 0., phi, c);
+        ae = c.ae;
+        aw = c.aw;
+        an = c.an;
+        as = c.as;
+        // the divisor as divk_make scales and inverts it, per lane
+        bool f;
+        s = __builtin_amdgcn_div_scale(1.0, ap, false, &f);
+        const double r0 = __builtin_amdgcn_rcp(s);
+        const double r1 = __builtin_fma(r0, __builtin_fma(-s, r0, 1.0), r0);
+        r = __builtin_fma(r1, __builtin_fma(-s, r1, 1.0), r1);
+    }
+    __device__ __forceinline__ double update(const StepArgs &a, double b, double pc, double pW, double pE, double pS,
+                                             double pN) const {
+        const double num = (((b - (ae * pE)) - (aw * pW)) - (an * pN)) - (as * pS);
+        DivFast dv;
+        double d = dv(num, DivK{ap, s, r});
+        if (dv.slow) d = num / ap;
+        return (d * a.omega) + (pc * a.omega_c);
+    }
+};
+template <>
+struct Cell2<float> {
+    float ae, aw, an, as, rap;
+    template <bool FAST>
+    __device__ __forceinline__ void set(const PfGeom &g, const StepArgs &a, int i, int j, const float *PHI,
+                                        const double *phi) {
+        CoefT<float> c;
+        float ap;
+        sor32_coefs<2>(g, a, i, j, 0, PHI[pf_soff(g, i, j, 0)], PHI[pf_soff(g, i - 1, j, 0)],
+                       PHI[pf_soff(g, i + 1, j, 0)], PHI[pf_soff(g, i, j - 1, 0)], PHI[pf_soff(g, i, j + 1, 0)], 0.f,
+                       0.f, phi, (float)(a.dt / (a.dx * a.dx)), (float)(a.dt / (a.dy * a.dy)),
+                       (float)(a.dt / (a.dz * a.dz)), c, ap);
+        ae = c.ae;
+        aw = c.aw;
+        an = c.an;
+        as = c.as;
+        rap = __builtin_amdgcn_rcpf(ap);
+    }
+    __device__ __forceinline__ float update(const StepArgs &a, float b, float pc, float pW, float pE, float pS,
+                                            float pN) const {
+        const float om = (float)a.omega;
+        const float num = b - ae * pE - aw * pW - an * pN - as * pS;
+        return num * rap * om + pc * (1.f - om);
+    }
+};
+
+}  // namespace
+
+template <typename T, int Q, bool FAST, bool ODD>
+__global__ __launch_bounds__(R2T) void k_sor_resident2(Resident2<T> x) {
+    extern __shared__ __align__(16) char lds_raw[];
+    T *L = (T *)lds_raw;   // [colour][local row][slot]
+    __shared__ int dead_flag;
+    const lds_int dead = (lds_int)&dead_flag;
+    const PfGeom &g = x.g;
+    const StepArgs &a = x.a;
+    constexpr int B = Msg<T>::B;
+    const int H = g.H, n = g.n, K = x.pl.K, R = x.pl.R, NR = x.pl.rows, N = NR * H, halo = x.pl.whole ? 0 : 2 * K;
+    const int tid = (int)threadIdx.x;
+    const int v0 = (int)blockIdx.x * R + 1 - halo;   // the row held in local row 0 (before wrapping)
+    const int own = min(R, n - ((int)blockIdx.x * R));
+    auto jrow = [=](int r) __attribute__((always_inline)) {
+        const int v = v0 + r;
+        return v < 1 ? v + n : v > n ? v - n : v;
+    };
+    if (tid == 0) *dead = 0;
+
+    // p of the held rows, ghost columns among it
+    for (int e = tid; e < 2 * N; e += R2T) {
+        const int c = e >= N, f = e - c * N, r = f / H, h = f - r * H;
+        L[e] = x.X[(int64_t)c * g.HS + pf_hoff(g, h, jrow(r), 0)];
+    }
+    // this thread's cells: place in a colour of L, distance from the held rows' edge (-1: no
+    // cell), row wraps, right-hand side and coefficients
+    int at[Q], depth[2][Q], south[2][Q], north[2][Q];
+    bool own_row[Q], odd_row[Q];
+    T b[2][Q];
+    Cell2<T> k[2][Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int f = tid + q * R2T, r = f / H, h = f - r * H;
+        at[q] = f;
+        own_row[q] = r >= halo && r < halo + own;
+        odd_row[q] = jrow(min(r, NR - 1)) & 1;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            depth[c][q] = -1;
+            b[c][q] = T(0);
+            south[c][q] = north[c][q] = 0;
+            k[c][q] = Cell2<T>{};
+            if (f >= N) continue;
+            const int j = jrow(r), i = 2 * h + ((c + j) & 1);
+            if (i < 1 || i > g.m) continue;
+            depth[c][q] = x.pl.whole ? 2 * K : min(r, NR - 1 - r);
+            b[c][q] = x.R[pf_soff(g, i, j, 0)];
+            k[c][q].template set<FAST>(g, a, i, j, x.PHI, x.phi);
+            // a neighbouring row's cell has the other colour, or this one across the wrap of an odd n
+            const int rs = r > 0 ? r - 1 : NR - 1, rn = r < NR - 1 ? r + 1 : 0;
+            south[c][q] = ((i + jrow(rs)) & 1) * N + rs * H + h;
+            north[c][q] = ((i + jrow(rn)) & 1) * N + rn * H + h;
+        }
+    }
+    const rsrc inbox = __builtin_amdgcn_make_buffer_rsrc(x.inbox, 0, (int)((uint32_t)(8 * n) * (uint32_t)H * B), 0x27000);
+    double err = 0.;
+    __syncthreads();
+
+    const int rounds = (x.iters + K - 1) / K;
+    for (int t = 0; t < rounds; ++t) {
+        if (t > 0) {
+            // exchange t - 1: the rows on each side, four messages in flight per thread
+            const uint32_t seq = x.seq + (uint32_t)(t - 1);
+            const int par = ((t - 1) & 3) * 2 * n * H * B, items = 2 * halo * H * 2;
+            unsigned spin = 0;
+            for (int e0 = 0; e0 < items; e0 += 4 * R2T) {
+                uint32_t src[4];
+                int dst[4];
+                bool want[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int e = e0 + tid + u * R2T, lr = e / (2 * H), w = e - lr * (2 * H), c = w >= H, h = w - c * H;
+                    const int r = lr < halo ? lr : lr + NR - 2 * halo;
+                    const int j = jrow(r), i = 2 * h + ((c + j) & 1);
+                    want[u] = e < items && i >= 1 && i <= g.m;
+                    src[u] = want[u] ? (uint32_t)(((j - 1) * 2 + c) * H + h) * B : 0u;
+                    dst[u] = c * N + r * H + h;
+                }
+                while (want[0] || want[1] || want[2] || want[3]) {
+                    decltype(Msg<T>::get(inbox, 0u, 0)) m[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) m[u] = Msg<T>::get(inbox, src[u], par);
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        if (want[u] && Msg<T>::ok(m[u], seq)) {
+                            L[dst[u]] = Msg<T>::value(m[u]);
+                            want[u] = false;
+                        }
+                    if ((want[0] || want[1] || want[2] || want[3]) && give_up(spin, dead)) break;
+                }
+            }
+            __syncthreads();
+        }
+        const int its = min(K, x.iters - t * K);
+        for (int it = 0; it < its; ++it) {
+            auto half = [&](auto HT) __attribute__((always_inline)) {
+                constexpr int half_no = decltype(HT)::value;
+                auto with = [&](auto CT) __attribute__((always_inline)) {
+                    constexpr int C = decltype(CT)::value;
+                    const int lost = 2 * it + half_no + 1;   // rows of each side no longer exact
+                    const bool ghosts = half_no == 0 && t == 0 && it == 0;
+                    T pn[Q];
+                    bool on[Q];
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) {
+                        on[q] = depth[C][q] >= lost;
+                        if (!on[q]) continue;
+                        const int f = at[q], sh = odd_row[q] ? 1 - C : C;
+                        const T *O = L + (1 - C) * N + f;
+                        T pS = L[south[C][q]], pN = L[north[C][q]];
+                        if (ghosts) {
+                            const int r = f / H, j = jrow(r), i = 2 * (f - r * H) + sh;
+                            if (j == 1) pS = x.X[pf_soff(g, i, 0, 0)];
+                            if (j == n) pN = x.X[pf_soff(g, i, n + 1, 0)];
+                        }
+                        const T pc = L[C * N + f];
+                        pn[q] = k[C][q].update(a, b[C][q], pc, O[sh - 1], O[sh], pS, pN);
+                        if (own_row[q]) err = max_keep_nan(err, fabs((double)pn[q] - (double)pc));
+                    }
+                    if (ODD) __syncthreads();
+#pragma unroll
+                    for (int q = 0; q < Q; ++q)
+                        if (on[q]) L[C * N + at[q]] = pn[q];
+                    __syncthreads();
+                };
+                if (half_no == 0) with(std::integral_constant<int, 1>{});   // (i + j) odd first
+                else with(std::integral_constant<int, 0>{});
+            };
+            half(std::integral_constant<int, 0>{});
+            half(std::integral_constant<int, 1>{});
+        }
+        if (t + 1 < rounds && !x.pl.whole) {
+            const uint32_t seq = x.seq + (uint32_t)t;
+            const int par = (t & 3) * 2 * n * H * B;
+            for (int e = tid; e < 2 * own * H; e += R2T) {
+                const int lr = e / (2 * H), w = e - lr * (2 * H), c = w >= H, h = w - c * H, j = v0 + halo + lr;
+                Msg<T>::send(inbox, (uint32_t)(((j - 1) * 2 + c) * H + h) * B, par, L[c * N + (halo + lr) * H + h], seq);
+            }
+        }
+    }
+
+    // the owned rows and their periodic mirrors back to memory
+    for (int e = tid; e < 2 * own * H; e += R2T) {
+        const int lr = e / (2 * H), w = e - lr * (2 * H), c = w >= H, h = w - c * H, j = v0 + halo + lr;
+        const int i = 2 * h + ((c + j) & 1);
+        if (i < 1 || i > g.m) continue;
+        const T v = L[c * N + (halo + lr) * H + h];
+        x.X[pf_soff(g, i, j, 0)] = v;
+        if (j == n) x.X[pf_soff(g, i, 0, 0)] = v;
+        if (j == 1) x.X[pf_soff(g, i, n + 1, 0)] = v;
+    }
+    wave_max_to_slot(err, x.slots);
+    __syncthreads();
+    if (tid == 0 && *dead) *x.fail = 1;
+}
+
+bool resident2_plan(const PfGeom &g, int bc, int iters, Resident2Plan &pl) {
+    pl = Resident2Plan{};
+    if (g.dim != 2 || bc != PF_BC_UNIFORM || g.n < 3 || iters < 2) return false;
+    const char *e = std::getenv("PF_RESIDENT");
+    int fk = 0, fr = 0;
+    if (e && *e && std::sscanf(e, "%d,%d", &fk, &fr) != 2) return false;
+    const int64_t H = g.H;
+    if (8 * H * g.n * 16 >= ((int64_t)1 << 31)) return false;   // byte offsets into the inbox are 32-bit
+    double best = 1e300;
+    auto consider = [&](int K, int R, bool whole) {
+        const int64_t rows = whole ? g.n : R + 4 * K, q = (rows * H + R2T - 1) / R2T;
+        const int64_t blocks = whole ? 1 : (g.n + R - 1) / R;
+        if (q > R2Q || blocks > RESIDENT_CUS || (!whole && rows > g.n)) return;
+        if (!whole && (iters + K - 1) / K < (g.n % R ? 3 : 2)) return;
+        // us of a half-sweep and of an exchange, from the figures above
+        const double half = 0.22 + 0.19 * (double)q;
+        const double cost = whole ? 2 * half : 2 * half + (1.6 + 0.0002 * (double)(8 * K * H)) / K;
+        if (cost < best) {
+            best = cost;
+            pl = Resident2Plan{whole ? iters : K, whole ? g.n : R, (int)rows, (int)q, (int)blocks, whole ? 1 : 0};
+        }
+    };
+    if (fk > 0 && fr > 0) {
+        consider(std::min(fk, iters / 2), fr, fr >= g.n);
+    } else {
+        consider(1, g.n, true);
+        const int r0 = (g.n + RESIDENT_CUS - 1) / RESIDENT_CUS;
+        for (int R = r0; R < r0 + 8; ++R)
+            for (int K = 1; K <= std::min(8, iters / 2); ++K) consider(K, R, false);
+    }
+    return pl.blocks > 0;
+}
+int64_t resident2_inbox_words(const PfGeom &g, int elem) { return (int64_t)8 * g.n * g.H * (elem == 8 ? 2 : 1); }
+
+template <typename T, int Q, bool FAST>
+static hipError_t run_resident2(hipStream_t st, Resident2<T> &r) {
+    const size_t lds = (size_t)2 * r.pl.rows * r.g.H * sizeof(T);
+    const void *f = (r.g.n & 1) ? (const void *)k_sor_resident2<T, Q, FAST, true> : (const void *)k_sor_resident2<T, Q, FAST, false>;
+    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    void *args[] = {&r};
+    if (r.pl.blocks == 1) return hipLaunchKernel(f, dim3(1), dim3(R2T), args, lds, st);
+    return hipLaunchCooperativeKernel(f, dim3((unsigned)r.pl.blocks), dim3(R2T), args, (unsigned)lds, st);
+}
+
+template <typename T>
+hipError_t launch_resident2(hipStream_t st, const PfGeom &g, const StepArgs &a, const Resident2Plan &pl, int iters,
+                            uint32_t seq, T *X, const T *R, const T *PHI, const double *phi, bool fast,
+                            unsigned long long *inbox, unsigned long long *slots, unsigned long long *fail) {
+    Resident2<T> r{g, a, pl, iters, seq, X, R, PHI, phi, inbox, slots, fail};
+#define PF_R2(QQ)                                                                      \
+    case QQ:                                                                           \
+        return fast ? run_resident2<T, QQ, true>(st, r) : run_resident2<T, QQ, false>(st, r);
+    switch (pl.q) {
+        PF_R2(1)
+        PF_R2(2)
+        PF_R2(3)
+        PF_R2(4)
+        PF_R2(5)
+        default: return hipErrorInvalidValue;
+    }
+#undef PF_R2
+}
+template hipError_t launch_resident2<double>(hipStream_t, const PfGeom &, const StepArgs &, const Resident2Plan &, int,
+                                             uint32_t, double *, const double *, const double *, const double *, bool,
+                                             unsigned long long *, unsigned long long *, unsigned long long *);
+template hipError_t launch_resident2<float>(hipStream_t, const PfGeom &, const StepArgs &, const Resident2Plan &, int,
+                                            uint32_t, float *, const float *, const float *, const double *, bool,
+                                            unsigned long long *, unsigned long long *, unsigned long long *);
+
 }  // namespace pf

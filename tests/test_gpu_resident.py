@@ -74,3 +74,69 @@ def test_resident_fp32_solve_matches_sweeps(bc, size, tiles, iters, monkeypatch)
             out[mode == "0"] = [s.interior(f) for f in ("u", "v", "w", "p")] + [st["sor_error"]]
     for a, b in zip(out[True], out[False]):
         np.testing.assert_array_equal(a, b)
+
+
+RUNS_2D = [
+    ((48, 24), "", 9),           # one block holds the grid
+    ((48, 23), "", 9),           # the same with an odd extent in y
+    ((37, 12), "1,2", 7),        # two rows a block, an exchange per iteration
+    ((37, 13), "1,2", 7),        # odd extent, the last block one row short
+    ((130, 40), "2,3", 9),       # two iterations between exchanges, ragged last block and round
+    ((131, 41), "3,1", 10),
+    ((97, 51), "", 40),
+    ((511, 255), "", 12),
+    ((700, 300), "", 5),
+    ((64, 32), "4,1", 8),        # as few rounds as a resident solve takes
+]
+
+
+@pytest.mark.parametrize("size,plan,iters", RUNS_2D)
+@pytest.mark.parametrize("step", [False, True])
+def test_resident_2d_solve_matches_oracle(size, plan, iters, step, monkeypatch):
+    import pyoracle
+    from pixelflow_amd.solver import Solver
+    if plan:
+        monkeypatch.setenv("PF_RESIDENT", plan)
+    print(f"[gpu] resident 2D {size} plan={plan or 'rule'} iters={iters} step={step}", flush=True)
+    p, phi = _case_2d(size, iters, 3, step)
+    o = pyoracle.OracleRun(p, phi)
+    ref = o.step(3)
+    with Solver(p, phi) as s:
+        st = s.step(3)
+        for f in ("u", "v", "p"):
+            np.testing.assert_array_equal(s.interior(f), o.interior(f), err_msg=f)
+        np.testing.assert_array_equal(st["sor_error"], ref)
+
+
+@pytest.mark.parametrize("size,plan,iters", RUNS_2D)
+def test_resident_2d_fp32_solve_matches_sweeps(size, plan, iters, monkeypatch):
+    """Also from ghost rows that are no mirrors of the grid's own (an uploaded pressure)."""
+    from pixelflow_amd.solver import PF_PREC_FP64, PF_PREC_MIXED, Solver
+    p, phi = _case_2d(size, iters, 3, False)
+    for prec in (PF_PREC_MIXED, PF_PREC_FP64):
+        out = {}
+        for mode in ("0", plan):
+            if mode:
+                monkeypatch.setenv("PF_RESIDENT", mode)
+            else:
+                monkeypatch.delenv("PF_RESIDENT")
+            monkeypatch.setenv("PF_SOR_TB2", "0,0") if mode == "0" else monkeypatch.delenv("PF_SOR_TB2")
+            print(f"[gpu] resident 2D sweeps {size} plan={mode or 'rule'} prec={prec}", flush=True)
+            with Solver(p, phi, precision=prec, inner_iters=iters if prec == PF_PREC_MIXED else 0) as s:
+                s.set_field("p", np.random.default_rng(3).standard_normal(p.full_shape()))
+                st = s.step(3)
+                out[mode == "0"] = [s.interior(f) for f in ("u", "v", "p")] + [st["sor_error"]]
+        for a, b in zip(out[True], out[False]):
+            np.testing.assert_array_equal(a, b)
+
+
+def _case_2d(size, iters, steps, step):
+    m, n = size
+    dx = 0.01
+    p = cases.CaseParams(dim=2, m=m, n=n, width=dx * (m - 1), height=dx * (n - 1), time=1e-4 * steps, istep_max=steps,
+                         iter_max=iters, inlet_porosity=step)
+    rng = np.random.default_rng(m * n)
+    phi = np.ones((n, m))
+    some = rng.random(phi.shape) < 0.1
+    phi[some] = rng.uniform(0.0, 1.0, int(some.sum()))
+    return p, phi
