@@ -150,6 +150,8 @@ struct MgSolver {
     bool own_mem = false;            // mem came from hipMalloc (else from the caller)
     int64_t bytes = 0;
     bool built = false;              // coarse operators match the current porosity
+    hipGraphExec_t gexec = nullptr;  // one iteration's kernels, for solves of several cases
+    bool graph_failed = false;
     // state of the current step's solve (mg_step_solve)
     int state = 0, cyc = 0, it = 0, vcycles = 0;
     double res = -1., b2 = 0.;

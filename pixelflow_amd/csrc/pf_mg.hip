@@ -1279,7 +1279,15 @@ bool mg_create(MgSolver<T> &S, const MgCase &c, std::string *why, void *mem) {
 }
 
 template <typename T>
+static void drop_graph(MgSolver<T> &S) {
+    if (S.gexec) (void)hipGraphExecDestroy(S.gexec);
+    S.gexec = nullptr;
+    S.graph_failed = false;
+}
+
+template <typename T>
 void mg_destroy(MgSolver<T> &S) {
+    drop_graph(S);
     if (S.mem && S.own_mem) (void)hipFree(S.mem);
     if (S.h_scal) (void)hipHostFree(S.h_scal);
     if (S.ev) (void)hipEventDestroy(S.ev);
@@ -1637,8 +1645,9 @@ static void enqueue_init(MgSolver<T> &S, hipStream_t st) {
     (void)hipMemcpyAsync(S.h_scal, S.scal, 8 * sizeof(double), hipMemcpyDeviceToHost, st);
 }
 
+// The kernels of one BiCGStab iteration (two V-cycles, over a hundred launches).
 template <typename T>
-static void enqueue_iteration(MgSolver<T> &S, hipStream_t st) {
+static void launch_iteration(MgSolver<T> &S, hipStream_t st) {
     const int64_t n = 2 * S.c.g.HS;
     const unsigned fb = flat_blocks(n);
     const int nap = (int)apply_blocks<T>(S.c.g);
@@ -1655,6 +1664,40 @@ static void enqueue_iteration(MgSolver<T> &S, hipStream_t st) {
     hipLaunchKernelGGL((k_bicg_xr<T>), dim3(fb), dim3(256), 0, st, n, S.x, (const T *)S.y, (const T *)S.z, S.r,
                        (const T *)S.s, (const T *)S.t, (const T *)S.rh, (const double *)S.scal, S.part);
     hipLaunchKernelGGL(k_bicg_scalar, dim3(1), dim3(256), 0, st, (const double *)S.part, (int)fb, S.scal, 3);
+}
+
+// The iteration as a graph: kernels only, every argument fixed until the next mg_setup.
+template <typename T>
+static bool iteration_graph(MgSolver<T> &S, hipStream_t st) {
+    if (S.gexec) return true;
+    if (S.graph_failed) return false;
+    S.graph_failed = true;
+    // relaxed: other threads' calls are none of this capture's concern
+    if (hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    launch_iteration(S, st);
+    hipGraph_t graph = nullptr;
+    hipError_t e = hipStreamEndCapture(st, &graph);
+    if (e == hipSuccess && graph) e = hipGraphInstantiate(&S.gexec, graph, nullptr, nullptr, 0);
+    if (graph) (void)hipGraphDestroy(graph);
+    if (e != hipSuccess || !S.gexec) {
+        (void)hipGetLastError();
+        S.gexec = nullptr;
+        return false;
+    }
+    S.graph_failed = false;
+    return true;
+}
+
+// shared: other solvers advance on other streams meanwhile.  Their launches come from this
+// one host thread, which at 3 to 4 us a launch kept up with little more than one of them:
+// there the iteration is one graph launch.  A solver alone is bound by the device's launch
+// boundary, which a graph does not shorten, and keeps its launches.
+template <typename T>
+static void enqueue_iteration(MgSolver<T> &S, hipStream_t st, bool shared) {
+    if (!(shared && iteration_graph(S, st) && hipGraphLaunch(S.gexec, st) == hipSuccess)) launch_iteration(S, st);
     (void)hipMemcpyAsync(S.h_scal, S.scal, 8 * sizeof(double), hipMemcpyDeviceToHost, st);
     S.vcycles += 2;
 }
@@ -1678,7 +1721,10 @@ hipError_t mg_step_solve(const std::vector<MgSolver<T> *> &runs, const std::vect
     for (size_t q = 0; q < nr; ++q) {
         MgSolver<T> &S = *runs[q];
         hipStream_t st = streams[q % ns];
-        if (!S.built) mg_setup(S, st);
+        if (!S.built) {
+            drop_graph(S);
+            mg_setup(S, st);
+        }
         S.state = MG_RESIDUAL;
         S.cyc = 0;
         S.it = 0;
@@ -1713,14 +1759,14 @@ hipError_t mg_step_solve(const std::vector<MgSolver<T> *> &runs, const std::vect
                     enqueue_update_and_residual(S, st);   // e = 0: the residual is re-read
                 } else {
                     S.it = 0;
-                    enqueue_iteration(S, st);
+                    enqueue_iteration(S, st, nr > 1);
                     S.state = MG_ITER;
                 }
             } else {   // MG_ITER
                 ++S.it;
                 const double rel = std::sqrt(S.h_scal[5] / S.b2);
                 if (!(rel > ctl.rtol) || S.h_scal[6] != 0. || S.it >= ctl.maxit) enqueue_update_and_residual(S, st);
-                else enqueue_iteration(S, st);
+                else enqueue_iteration(S, st, nr > 1);
             }
             if ((err = hipEventRecord(S.ev, st)) != hipSuccess) return err;
         }
