@@ -10,7 +10,10 @@ One "step" is one time step: predictor, Poisson RHS, 100 SOR iterations (200 col
 sweeps), projection and boundary update, all resident in HBM.  The line printed:
 
   value       cell-steps/s = m*n*l*steps / wall seconds of the timed steps
-  roofline    the SOR colour-sweep kernel: algorithmic bytes per launch (3 FP64 words per
+  roofline    the kernel of the pressure solve.  Where it keeps the grid on chip (the default
+              workload): FP64 operations against the vector peak without FMA, with the same
+              steps by one launch per colour sweep under `streamed`.  Else the SOR
+              colour-sweep kernel: algorithmic bytes per launch (3 FP64 words per
               cell: read p, write p of half the cells, read bb of half, read porosity --
               the streamed model 8*(2d+2 + 6K + 2d+1) B per cell-step) / average launch
               time measured with HIP events on the solver's stream; traffic = measured
@@ -216,6 +219,45 @@ def cpu_baseline_one_thread(m: int, n: int, l: int, steps: int):
     return v[0], v[1]
 
 
+FP64_PEAK_GFLOPS = 78600.0   # vector FP64, FMA counted as two
+SOR_FLOPS = 24               # FP64 instructions of one update of a unit-porosity cell
+
+
+def resident_roofline(kernel: str, launch_us: float, cells: int, iters: int, unit: int):
+    """The resident solve moves its bytes once a step; what bounds it is FP64 issue of the
+    fullest tile and the exchange of tile surfaces, so its rate is given in FP64 operations
+    (one per instruction: there is no FMA in the reference's arithmetic)."""
+    achieved = cells * iters * SOR_FLOPS / (launch_us * 1e-6) / 1e9
+    return {"bound": "fp64 issue and the exchange between tiles", "kernel": kernel, "achieved": achieved,
+            "peak": FP64_PEAK_GFLOPS / 2, "unit": "GFLOP/s", "frac": achieved / (FP64_PEAK_GFLOPS / 2),
+            "bytes_per_launch_algorithmic": 3 * 8 * cells, "avg_launch_us": launch_us,
+            "avg_half_sweep_us": launch_us / (2 * iters), "unit_porosity_cells": unit}
+
+
+def streamed_sweep(p, phi, steps: int, workload: str):
+    """The same steps with one launch per colour sweep (PF_RESIDENT=0), and that kernel's
+    roofline: 3 FP64 words per grid cell and launch, less one per cell of a unit-porosity wave."""
+    from pixelflow_amd.solver import Solver
+    saved = os.environ.get("PF_RESIDENT")
+    os.environ["PF_RESIDENT"] = "0"
+    try:
+        with Solver(p, phi) as s:
+            wall, us, _ = _timed_run(s, steps, 2)
+            unit = s.sor_unit_cells()
+    finally:
+        if saved is None:
+            os.environ.pop("PF_RESIDENT", None)
+        else:
+            os.environ["PF_RESIDENT"] = saved
+    bytes_ = 24 * p.cells - 8 * unit
+    achieved = bytes_ / (us * 1e-6) / 1e9
+    return {"ms_per_step": wall * 1e3 / steps, "steps": steps,
+            "roofline": {"bound": "hbm", "kernel": "k_sor_phi (red/black colour sweep)", "achieved": achieved,
+                         "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
+                         "traffic": measured_traffic("k_sor_phi", workload), "bytes_per_launch_algorithmic": bytes_,
+                         "avg_launch_us": us, "unit_porosity_cells": unit}}
+
+
 def mixed_comparison(p, phi, steps: int, warmup: int, inner: int, fp64_value: float):
     """Same workload in mixed precision (fixed-count mode: the reference's iter_max), timed,
     then the fields after `steps` steps compared with an FP64 run of the same steps."""
@@ -232,6 +274,7 @@ def mixed_comparison(p, phi, steps: int, warmup: int, inner: int, fp64_value: fl
     wall = time.perf_counter() - t0
     sweep_us, _ = b.last_sweep_time_us()
     unit = b.sor_unit_cells()
+    resident = b.sor_resident()
     a = Solver(p, phi)
     a.step(warmup + steps)
     errs = {}
@@ -243,11 +286,13 @@ def mixed_comparison(p, phi, steps: int, warmup: int, inner: int, fp64_value: fl
     b.close()
     v = p.cells * steps / wall
     # mixed bytes per cell-iteration: 2 FP32 half-sweeps of 3 words (less 2 words per cell of
-    # a unit-porosity wave over the two: its own porosity and its neighbours'), per cycle an
+    # a unit-porosity wave over the two: its own porosity and its neighbours'; a resident solve
+    # reads e and r and writes e once per cycle), per cycle an
     # FP64 residual (p 8, bb 8, porosity 8 read, r 4 + e 4 written) and an update (e 4, p 8 + 8)
     K = inner or p.iter_max
     cyc = (p.iter_max + K - 1) // K
-    solve_bytes = p.cells * (p.iter_max * 2 * 3 * 4 + cyc * (8 * 3 + 4 + 4 + 4 + 16)) - p.iter_max * 8 * unit
+    sweep_bytes = 3 * 4 * p.cells * cyc if resident else p.cells * p.iter_max * 2 * 3 * 4 - p.iter_max * 8 * unit
+    solve_bytes = sweep_bytes + p.cells * cyc * (8 * 3 + 4 + 4 + 4 + 16)
     return {"value": v, "unit": "cell-steps/s", "ms_per_step": wall * 1e3 / steps, "steps": steps,
             "speedup_vs_fp64": v / fp64_value, "sor_cell_updates_per_s": v * p.iter_max,
             "inner_iters": K, "cycles_per_step": cyc, "avg_solve_us_per_iteration_half": sweep_us,
@@ -455,16 +500,21 @@ def main(argv=None):
     wall = time.perf_counter() - t0
     sweep_us, launches = s.last_sweep_time_us()
     fused = s.sor_fused()
+    resident = s.sor_resident()
     unit = s.sor_unit_cells()
     s.close()
     log(f"[bench] {args.steps} steps in {wall:.3f} s; colour sweep avg {sweep_us:.2f} us over {launches} sweeps"
-        f" ({'fused: one launch per iteration' if fused else 'one launch per colour sweep'})")
+        f" ({'one resident launch per step' if resident else 'fused: one launch per iteration' if fused else 'one launch per colour sweep'})")
     from pixelflow_amd.solver import probe_copy_gbps
     copy_gbps = {"128MB": probe_copy_gbps(128 << 20, 20), "2GB": probe_copy_gbps(2048 << 20, 10)}
 
     cells = p.cells
     value = cells * args.steps / wall
-    if fused:
+    if resident:
+        # one launch = a step's whole solve: p and bb read and p written once
+        kernel, launch_us, launch_bytes = ("k_sor_resident (a step's SOR iterations, the grid on chip)",
+                                           2 * p.iter_max * sweep_us, 3 * 8 * cells)
+    elif fused:
         # one launch = one red/black iteration: p read and written once, bb and porosity
         # read once (4 FP64 words per cell)
         kernel, launch_us, launch_bytes = "k_sor_fused (one red/black SOR iteration)", 2 * sweep_us, 4 * 8 * cells
@@ -475,8 +525,9 @@ def main(argv=None):
         # of either colour, in such waves
         kernel, launch_us, launch_bytes = "k_sor_phi (red/black colour sweep)", sweep_us, 3 * 8 * cells - 8 * unit
     achieved = launch_bytes / (launch_us * 1e-6) / 1e9 if launch_us > 0 else 0.0
-    sor_bytes = 4 * 8 * cells if fused else 2 * launch_bytes   # per SOR iteration
-    step_bytes = 8 * ((2 * 3 + 2) + (2 * 3 + 1)) * cells + sor_bytes * p.iter_max
+    # of a step's solve
+    sor_bytes = launch_bytes if resident else (4 * 8 * cells if fused else 2 * launch_bytes) * p.iter_max
+    step_bytes = 8 * ((2 * 3 + 2) + (2 * 3 + 1)) * cells + sor_bytes
     res = {
         "metric": METRIC,
         "value": value,
@@ -496,7 +547,7 @@ def main(argv=None):
         "step_roofline_frac": (step_bytes * args.steps / wall / 1e9) / HBM_PEAK_GBS,
         "final_sor_error": float(st["sor_error"][-1]),
         "device_copy_GBps": copy_gbps,
-        "roofline": {
+        "roofline": resident_roofline(kernel, launch_us, cells, p.iter_max, unit) if resident else {
             "bound": "hbm",
             "kernel": kernel,
             "achieved": achieved,
@@ -509,6 +560,8 @@ def main(argv=None):
             "unit_porosity_cells": unit,
         },
     }
+    if resident:
+        res["streamed"] = streamed_sweep(p, phi, min(args.steps, 50), workload)
     if args.mixed_steps > 0:
         res["mixed"] = mixed_comparison(p, phi, args.mixed_steps, args.warmup, args.mixed_inner, value)
     cpus = host_cpus()

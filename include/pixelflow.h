@@ -161,6 +161,9 @@ int pf_probe_copy(int64_t bytes, int iters, double *gbps);
  * buffers; even periodic extents; opt-in with PF_FUSED=1 in the environment), 0 if as two
  * colour-sweep launches (the default, faster on MI355X).  Same results. */
 int pf_sor_fused(const pf_ctx *ctx);
+/* 1 if the context solves a fixed count of SOR iterations as one launch that keeps the grid
+ * on chip, 0 if with a launch per colour sweep or per few iterations.  Same results. */
+int pf_sor_resident(const pf_ctx *ctx);
 /* 1 if the FP64 colour sweeps read the porosity coded in 4 bytes per value (values FP32
  * holds exactly as floats, the others through a table of at most 2^20 distinct doubles:
  * the same doubles, 4 fewer bytes per cell and sweep; the default past 512 MB of sweep

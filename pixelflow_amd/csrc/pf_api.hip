@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <string>
 #include <utility>
@@ -76,7 +77,9 @@ struct pf_ctx {
     uint32_t *rmask = nullptr, *rfirst = nullptr;
     unsigned long long *rinbox = nullptr;
     uint32_t rseq = 1;              // next unused message sequence number
-    unsigned long long *rfail = nullptr;   // set by a launch whose bounded wait ran out
+    unsigned long long *rcount = nullptr;  // blocks that finished, over all launches (device)
+    unsigned long long *rcount_host = nullptr;   // pinned copy
+    unsigned long long rtarget = 0;
     pf::Downloader down;
     int err_cap = 0, nparts = 0;
     bool have_phi = false, have_init = false;
@@ -122,7 +125,8 @@ static bool desc_ok(const pf_desc *d, std::string &why) { return pf::desc_valid(
 extern "C" int pf_abi_version(void) { return PF_ABI_VERSION; }
 
 // The temporally blocked 2D sweep's iterations per launch and rows per block, or 0 and 0
-// where it is not used: FP64, 2D, and the shape within what the kernel holds.  By default 2
+// where it is not used: FP64, 2D, and the shape within what the kernel holds, for contexts
+// whose solves are not resident (resident2_wanted).  By default 2
 // iterations and 1 row (on the 256x128 cylinder, ms per step: two-launch sweeps 0.86, K,R =
 // 1,1 0.60, 2,1 0.47, 2,2 0.54, 3,1 0.48, 4,1 0.52 with porosity in LDS, 4,8 0.80); rows
 // wider than about 310 cells do not fit LDS and keep the two-launch sweeps.
@@ -234,6 +238,8 @@ static void release(pf_ctx *c) {
     if (c->rmask) { (void)hipFree(c->rmask); c->rmask = nullptr; }
     if (c->rfirst) { (void)hipFree(c->rfirst); c->rfirst = nullptr; }
     if (c->rinbox) { (void)hipFree(c->rinbox); c->rinbox = nullptr; }
+    if (c->rcount) { (void)hipFree(c->rcount); c->rcount = nullptr; }
+    if (c->rcount_host) { (void)hipHostFree(c->rcount_host); c->rcount_host = nullptr; }
     if (c->mg32) { pf::mg_destroy(*c->mg32); delete c->mg32; c->mg32 = nullptr; }
     if (c->mg64) { pf::mg_destroy(*c->mg64); delete c->mg64; c->mg64 = nullptr; }
     for (hipEvent_t e : c->evs) (void)hipEventDestroy(e);
@@ -283,15 +289,18 @@ extern "C" int pf_create(const pf_desc *desc, pf_ctx **out) {
     }
     c->nparts = pf::sor_blocks(g);
     {
-        int cus = 0, coop = 0;
-        c->resident = resident_wanted(g, desc, c->rpl) &&
-                      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess &&
-                      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess &&
-                      coop && c->rpl.bx * c->rpl.by * c->rpl.bz <= cus;
-        c->resident2 = resident2_wanted(g, desc) &&
-                       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess &&
-                       hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess &&
-                       coop && cus >= pf::RESIDENT_CUS;
+        int cus = 0;
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess) cus = 0;
+        c->resident = resident_wanted(g, desc, c->rpl) && c->rpl.bx * c->rpl.by * c->rpl.bz <= cus;
+        c->resident2 = resident2_wanted(g, desc) && cus >= pf::RESIDENT_CUS;
+    }
+    if (c->resident || c->resident2) {
+        if (hipMalloc((void **)&c->rcount, 8) != hipSuccess ||
+            hipHostMalloc((void **)&c->rcount_host, 8, hipHostMallocDefault) != hipSuccess) {
+            rc = fail(c, PF_ENOMEM, "hipMalloc of the resident sweep's count failed");
+            goto bad;
+        }
+        pf::launch_clear_u64(c->st, c->rcount, 1);
     }
     if (c->resident2) {
         const int64_t words = pf::resident2_inbox_words(g, desc->precision == PF_PREC_MIXED ? 4 : 8);
@@ -661,6 +670,25 @@ extern "C" int pf_initial(pf_ctx *c) {
 // The time step
 // ------------------------------------------------------------------------------------
 // A solve of `iters` iterations as one resident launch; false where it does not apply.
+// What a resident launch of `blocks` blocks left: true with its result in place, false with
+// nothing changed (the half-sweep kernels take over).  Waits for the launch.
+static bool resident_done(pf_ctx *c, hipError_t e) {
+    if (e == hipSuccess) e = hipMemcpyAsync(c->rcount_host, c->rcount, 8, hipMemcpyDeviceToHost, c->st);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->st);
+    if (e == hipSuccess && *c->rcount_host == c->rtarget) return true;
+    (void)hipGetLastError();
+    // its blocks found no room beside other work on the GPU, or it could not be launched: this
+    // context stays with the half-sweep kernels
+    c->resident = c->resident2 = false;
+    return false;
+}
+// Resident launches of this process, one at a time per device: two at once would keep each
+// other's last blocks out until both gave up.
+static std::mutex &resident_lock(int device) {
+    static std::mutex locks[16];
+    return locks[(unsigned)device % 16u];
+}
+
 static bool enqueue_resident2(pf_ctx *c, unsigned long long *slot, int iters) {
     pf::Resident2Plan pl;
     if (!c->resident2 || c->fused || c->sor_variant == 0 || iters >= (1 << 28) ||
@@ -671,17 +699,21 @@ static bool enqueue_resident2(pf_ctx *c, unsigned long long *slot, int iters) {
         pf::launch_clear_u64(c->st, c->rinbox, (int)pf::resident2_inbox_words(c->g, f32 ? 4 : 8));
         c->rseq = 1;
     }
-    const hipError_t e = f32 ? pf::launch_resident2<float>(c->st, c->g, c->a, pl, iters, c->rseq, c->E32, c->R32, c->PHI32,
-                                                           c->phi, fast, c->rinbox, slot, c->rfail)
-                             : pf::launch_resident2<double>(c->st, c->g, c->a, pl, iters, c->rseq, c->P, c->BB, c->PHIs,
-                                                            c->phi, fast, c->rinbox, slot, c->rfail);
-    if (e != hipSuccess) {   // not launched: the half-sweep kernels take over
-        (void)hipGetLastError();
-        c->resident2 = false;
-        return false;
+    std::unique_lock<std::mutex> lock(resident_lock(c->device), std::defer_lock);
+    if (!pl.whole) {
+        lock.lock();
+        c->rtarget += (unsigned long long)pl.blocks;
     }
+    const hipError_t e = f32 ? pf::launch_resident2<float>(c->st, c->g, c->a, pl, iters, c->rseq, c->E32, c->R32, c->PHI32,
+                                                           c->phi, fast, c->rinbox, slot, c->rcount, c->rtarget)
+                             : pf::launch_resident2<double>(c->st, c->g, c->a, pl, iters, c->rseq, c->P, c->BB, c->PHIs,
+                                                            c->phi, fast, c->rinbox, slot, c->rcount, c->rtarget);
     c->rseq += (uint32_t)iters;
-    return true;
+    if (!pl.whole) return resident_done(c, e);
+    if (e == hipSuccess) return true;   // one block waits for nobody
+    (void)hipGetLastError();
+    c->resident2 = false;
+    return false;
 }
 static bool enqueue_resident(pf_ctx *c, unsigned long long *slot, int iters) {
     if (c->g.dim == 2) return enqueue_resident2(c, slot, iters);
@@ -692,18 +724,15 @@ static bool enqueue_resident(pf_ctx *c, unsigned long long *slot, int iters) {
         pf::launch_clear_u64(c->st, c->rinbox, (int)pf::resident_inbox_words(c->rpl, f32 ? 4 : 8));
         c->rseq = 1;
     }
+    std::lock_guard<std::mutex> lock(resident_lock(c->device));
+    c->rtarget += (unsigned long long)(c->rpl.bx * c->rpl.by * c->rpl.bz);
     const hipError_t e =
         f32 ? pf::launch_resident<float>(c->st, c->g, c->a, c->rpl, iters, c->rseq, c->E32, c->R32, (const float *)c->rcoef,
-                                         c->rmask, c->rfirst, c->rinbox, slot, c->rfail)
+                                         c->rmask, c->rfirst, c->rinbox, slot, c->rcount, c->rtarget)
             : pf::launch_resident<double>(c->st, c->g, c->a, c->rpl, iters, c->rseq, c->P, c->BB, (const double *)c->rcoef,
-                                          c->rmask, c->rfirst, c->rinbox, slot, c->rfail);
-    if (e != hipSuccess) {   // not launched: the half-sweep kernels take over
-        (void)hipGetLastError();
-        c->resident = false;
-        return false;
-    }
+                                          c->rmask, c->rfirst, c->rinbox, slot, c->rcount, c->rtarget);
     c->rseq += 2u * (uint32_t)iters;
-    return true;
+    return resident_done(c, e);
 }
 
 static void enqueue_sor(pf_ctx *c, unsigned long long *slot, int iters) {
@@ -918,11 +947,10 @@ extern "C" int pf_step(pf_ctx *c, int nsteps, pf_stats *stats) {
     if (c->err_cap < nsteps) {
         if (c->err) PF_TRY_HIP(c, hipFree(c->err));
         c->err = nullptr;
-        PF_TRY_HIP(c, hipMalloc((void **)&c->err, sizeof(unsigned long long) * ((size_t)nsteps + 1)));
+        PF_TRY_HIP(c, hipMalloc((void **)&c->err, sizeof(unsigned long long) * (size_t)nsteps));
         c->err_cap = nsteps;
     }
-    pf::launch_clear_u64(c->st, c->err, nsteps + 1);
-    c->rfail = c->err + nsteps;
+    pf::launch_clear_u64(c->st, c->err, nsteps);
     c->mixed_res.clear();
     c->mixed_cycles.clear();
     c->mixed_iters.clear();
@@ -969,11 +997,9 @@ extern "C" int pf_step(pf_ctx *c, int nsteps, pf_stats *stats) {
         pf::launch_boundary(c->st, g, c->a, c->phi, c->u, c->v, c->w, c->P);
         PF_TRY_HIP(c, hipGetLastError());
     }
-    std::vector<unsigned long long> e((size_t)nsteps + 1);
+    std::vector<unsigned long long> e((size_t)nsteps);
     PF_TRY_HIP(c, hipMemcpyAsync(e.data(), c->err, sizeof(unsigned long long) * e.size(), hipMemcpyDeviceToHost, c->st));
     PF_TRY_HIP(c, hipStreamSynchronize(c->st));
-    if (e[(size_t)nsteps] != 0)
-        return fail(c, PF_EHIP, "resident sweep: a tile's wait for its neighbours ran out (PF_RESIDENT=0 avoids it)");
     if (c->timing && c->d.iter_max > 0) {
         double sweep_ms = 0.0;
         for (int s = 0; s < nsteps; ++s) {
@@ -1045,6 +1071,12 @@ extern "C" int pf_sor_fused(const pf_ctx *c) {
     if (!c) return PF_EINVAL;
     if (!c->fused) return 0;
     return (c->d.precision == PF_PREC_MIXED || c->sor_variant != 0) ? 1 : 0;
+}
+
+extern "C" int pf_sor_resident(const pf_ctx *c) {
+    if (!c) return PF_EINVAL;
+    if (c->fused || c->sor_variant == 0 || !c->have_phi) return 0;
+    return ((c->resident && c->rcoef) || c->resident2) ? 1 : 0;
 }
 
 extern "C" int pf_set_timing(pf_ctx *c, int on) {

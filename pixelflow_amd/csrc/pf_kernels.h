@@ -132,10 +132,13 @@ void launch_resident_setup(hipStream_t st, const PfGeom &g, const StepArgs &a, c
                            const double *phi, T *coef, uint32_t *mask, const uint32_t *first, bool fast);
 // iters red/black iterations, even cells first, on X (colour-split, ghosts current) with right-hand side R.
 // Half-sweep h's messages carry seq + h, which no earlier launch on this inbox may have used.
+// The result is there if *count is target afterwards: the number of blocks of all launches on
+// it, this one's included.  Else X and the slots are as before, and *count has its top bit set.
 template <typename T>
 hipError_t launch_resident(hipStream_t st, const PfGeom &g, const StepArgs &a, const ResidentPlan &pl, int iters,
                            uint32_t seq, T *X, const T *R, const T *coef, const uint32_t *mask, const uint32_t *first_set,
-                           unsigned long long *inbox, unsigned long long *slots, unsigned long long *fail);
+                           unsigned long long *inbox, unsigned long long *slots, unsigned long long *count,
+                           unsigned long long target);
 // The same in 2D: K iterations between exchanges, R rows a block, `rows` held, q cells of each
 // colour a thread, whole: one block holds the grid.  PF_RESIDENT="K,R" in the environment
 // sets them ("0": never).
@@ -148,7 +151,8 @@ int64_t resident2_inbox_words(const PfGeom &g, int elem);
 template <typename T>
 hipError_t launch_resident2(hipStream_t st, const PfGeom &g, const StepArgs &a, const Resident2Plan &pl, int iters,
                             uint32_t seq, T *X, const T *R, const T *PHI, const double *phi, bool fast,
-                            unsigned long long *inbox, unsigned long long *slots, unsigned long long *fail);
+                            unsigned long long *inbox, unsigned long long *slots, unsigned long long *count,
+                           unsigned long long target);
 // Body force (pressure + wall-force terms): partial holds force_blocks(g)*6 doubles, out 6.
 int force_blocks(const PfGeom &g);
 void launch_force(hipStream_t st, const PfGeom &g, const StepArgs &a, const double *phi, const double *u,

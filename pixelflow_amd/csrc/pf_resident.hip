@@ -15,9 +15,13 @@
 // parity.  A block writes a slot again two iterations later, when it has received
 // messages that its neighbour sent after reading the slot.
 //
-// Waiting.  The launch is cooperative: all blocks are resident together, one per CU.  A
-// block waits only for its face neighbours' previous half-sweep, and a wait ends after a
-// bounded number of polls with *fail set.
+// Waiting.  The blocks need each other and are at most one per CU, but the launch is an
+// ordinary one: after a cooperative launch the process's other streams ran one after the
+// other (16 rooms on three streams 150 -> 270 ms a step).  So nothing rests on their being
+// resident together.  Every wait ends after a bounded number of polls; then, or as soon as
+// another block has given up, a block leaves without a trace: results are written only after
+// all blocks have counted themselves in at the end (commit).  The host looks at the count
+// after the launch and runs the per-half-sweep kernels where it came to nothing.
 //
 // Arithmetic.  Per cell the operations and their order are those of sor_value (FP64) and
 // sor32_value (FP32), on the same operands: a cell whose seven porosities are 1 takes the
@@ -51,7 +55,6 @@ constexpr int RT = 32;              // widest tile in x and y
 constexpr int RP = RT + 2;          // LDS pitch of a plane with its halo
 constexpr int RPL = RP * RP;
 constexpr int RMAXT = 1024;         // threads of a block, one per column of the tile
-constexpr unsigned RSPIN = 1u << 22;
 
 typedef unsigned long long u64;
 
@@ -223,7 +226,8 @@ struct ResidentRun {
     const uint32_t *mask, *first;
     u64 *inbox;
     u64 *slots;
-    u64 *fail;
+    u64 *count, target;   // blocks that reached the end, over all launches: target with this one's
+    unsigned polls;       // of a wait, at most
 };
 
 using lds_int = __attribute__((address_space(3))) volatile int *;
@@ -243,6 +247,8 @@ struct Work {
     DivK kap;
     T *L;
     lds_int dead;
+    u64 *count;
+    unsigned polls;
     // the column
     T b[2][NS];             // right-hand side by colour and height pair: cell (c, s) lies at z = 2s + q(c)
     T zlo, zhi;             // the cells below and above the column
@@ -299,11 +305,38 @@ __device__ __forceinline__ bool side_item(const Work<T, NS> &w, int e, int cc, u
     return nb >= 0 && z < t.hz;
 }
 
+constexpr u64 GONE = 1ull << 63;   // in the commit count: a block has given up
+
+__device__ __forceinline__ u64 count_now(u64 *count) {
+    return __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // One more poll without success: true when the wait is over without its message.
-__device__ __forceinline__ bool give_up(unsigned &spin, lds_int dead) {
-    if (++spin < RSPIN && !*dead) return false;
+__device__ __forceinline__ bool give_up(unsigned &spin, lds_int dead, u64 *count, unsigned polls) {
+    ++spin;
+    if (spin < polls && !*dead && ((spin & 255u) || !(count_now(count) & GONE))) return false;
     *dead = 1;
     return true;
+}
+
+// The end of a block (one thread): true when every block of the launch has come here, which
+// brings the count to `target`, and none had given up before.  The two are decided by the
+// one word, so all blocks get the same answer.
+__device__ __forceinline__ bool commit(u64 *count, u64 target, bool dead, unsigned polls) {
+    if (!dead) (void)__hip_atomic_fetch_add(count, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    u64 v = count_now(count);
+    for (unsigned spin = 0; !dead && spin < polls; ++spin) {
+        if (v & GONE) return false;
+        if (v >= target) return true;
+        v = count_now(count);
+    }
+    while (!(v & GONE)) {
+        if (v >= target) return true;
+        if (__hip_atomic_compare_exchange_strong(count, &v, v | GONE, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT))
+            return false;
+    }
+    return false;
 }
 
 // Half-sweep h, of colour C.
@@ -336,7 +369,7 @@ __device__ __forceinline__ void half_sweep(Work<T, NS> &w, int h) {
             if (w0 && Msg<T>::ok(m0, seq)) { w.zlo = Msg<T>::value(m0); w0 = false; }
             if (w1 && Msg<T>::ok(m1, seq)) { w.zhi = Msg<T>::value(m1); w1 = false; }
             if (w2 && Msg<T>::ok(m2, seq)) { w.L[sd] = Msg<T>::value(m2); w2 = false; }
-            if ((w0 || w1 || w2) && give_up(spin, w.dead)) break;
+            if ((w0 || w1 || w2) && give_up(spin, w.dead, w.count, w.polls)) break;
         }
         for (int e = w.tid + w.nthr; e < w.nside; e += w.nthr) {
             uint32_t src;
@@ -344,7 +377,7 @@ __device__ __forceinline__ void half_sweep(Work<T, NS> &w, int h) {
             if (!side_item<T, NS>(w, e, O, src, dst)) continue;
             auto m = Msg<T>::get(w.inbox, src, in);
             while (!Msg<T>::ok(m, seq)) {
-                if (give_up(spin, w.dead)) break;
+                if (give_up(spin, w.dead, w.count, w.polls)) break;
                 m = Msg<T>::get(w.inbox, src, in);
             }
             w.L[dst] = Msg<T>::value(m);
@@ -440,6 +473,8 @@ __global__ __launch_bounds__(RMAXT) void k_sor_resident(ResidentRun<T> r) {
     const int bx = r.pl.bx, by = r.pl.by, bz = r.pl.bz;
     if (tid == 0) dead = 0;
     w.dead = (lds_int)&dead;
+    w.count = r.count;
+    w.polls = r.polls;
     w.L = L;
     w.gm = r.g.m;
     w.gn = r.g.n;
@@ -547,6 +582,11 @@ __global__ __launch_bounds__(RMAXT) void k_sor_resident(ResidentRun<T> r) {
         half_sweep<T, NS, 1, ODDY>(w, h + 1);
     }
 
+    __syncthreads();
+    if (tid == 0) dead = commit(r.count, r.target, dead != 0, r.polls) ? 0 : 1;
+    __syncthreads();
+    if (dead) return;
+
     // the column and its periodic mirrors back to memory
     if (t.act) {
 #pragma unroll
@@ -566,13 +606,19 @@ __global__ __launch_bounds__(RMAXT) void k_sor_resident(ResidentRun<T> r) {
             }
     }
     wave_max_to_slot(w.err, r.slots);
-    __syncthreads();
-    if (tid == 0 && dead) *r.fail = 1;
 }
 
 // ------------------------------------------------------------------------------------
 // Host side
 // ------------------------------------------------------------------------------------
+// Polls of a wait, at most: about 0.4 s of them.  PF_RESIDENT_POLLS in the environment sets
+// another number (tests: 1 makes launches give up).
+static unsigned resident_polls() {
+    const char *e = std::getenv("PF_RESIDENT_POLLS");
+    const int v = (e && *e) ? std::atoi(e) : 0;
+    return v > 0 ? (unsigned)v : 1u << 19;
+}
+
 static int ns_of(int tz) {
     const int h = (tz + 1) / 2;
     return h <= 1 ? 1 : h <= 2 ? 2 : h <= 4 ? 4 : h <= 8 ? 8 : 16;
@@ -637,8 +683,7 @@ static hipError_t run_resident(hipStream_t st, ResidentRun<T> &r) {
     const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     void *args[] = {&r};
-    return hipLaunchCooperativeKernel(f, dim3((unsigned)(r.pl.bx * r.pl.by * r.pl.bz)), dim3((unsigned)r.pl.threads),
-                                      args, (unsigned)lds, st);
+    return hipLaunchKernel(f, dim3((unsigned)(r.pl.bx * r.pl.by * r.pl.bz)), dim3((unsigned)r.pl.threads), args, lds, st);
 }
 template <typename T, int NS>
 static hipError_t run_resident(hipStream_t st, ResidentRun<T> &r) {
@@ -649,8 +694,9 @@ static hipError_t run_resident(hipStream_t st, ResidentRun<T> &r) {
 template <typename T>
 hipError_t launch_resident(hipStream_t st, const PfGeom &g, const StepArgs &a, const ResidentPlan &pl, int iters,
                            uint32_t seq, T *X, const T *R, const T *coef, const uint32_t *mask, const uint32_t *first_set,
-                           unsigned long long *inbox, unsigned long long *slots, unsigned long long *fail) {
-    ResidentRun<T> r{g, a, pl, iters, seq, X, R, coef, mask, first_set, inbox, slots, fail};
+                           unsigned long long *inbox, unsigned long long *slots, unsigned long long *count,
+                            unsigned long long target) {
+    ResidentRun<T> r{g, a, pl, iters, seq, X, R, coef, mask, first_set, inbox, slots, count, target, resident_polls()};
     switch (pl.ns) {
         case 1: return run_resident<T, 1>(st, r);
         case 2: return run_resident<T, 2>(st, r);
@@ -664,11 +710,13 @@ hipError_t launch_resident(hipStream_t st, const PfGeom &g, const StepArgs &a, c
 template hipError_t launch_resident<double>(hipStream_t, const PfGeom &, const StepArgs &, const ResidentPlan &, int,
                                             uint32_t, double *, const double *, const double *, const uint32_t *,
                                             const uint32_t *,
-                                            unsigned long long *, unsigned long long *, unsigned long long *);
+                                            unsigned long long *, unsigned long long *, unsigned long long *,
+                                            unsigned long long);
 template hipError_t launch_resident<float>(hipStream_t, const PfGeom &, const StepArgs &, const ResidentPlan &, int,
                                            uint32_t, float *, const float *, const float *, const uint32_t *,
                                            const uint32_t *,
-                                           unsigned long long *, unsigned long long *, unsigned long long *);
+                                           unsigned long long *, unsigned long long *, unsigned long long *,
+                                            unsigned long long);
 
 template <typename T, int NS>
 static void run_resident_setup(hipStream_t st, const PfGeom &g, const StepArgs &a, const ResidentPlan &pl, const T *PHI,
@@ -736,7 +784,8 @@ struct Resident2 {
     const double *phi;
     u64 *inbox;
     u64 *slots;
-    u64 *fail;
+    u64 *count, target;   // blocks that reached the end, over all launches: target with this one's
+    unsigned polls;       // of a wait, at most
 };
 
 // A cell's coefficients and what its division needs.
@@ -888,7 +937,7 @@ __global__ __launch_bounds__(R2T) void k_sor_resident2(Resident2<T> x) {
                             L[dst[u]] = Msg<T>::value(m[u]);
                             want[u] = false;
                         }
-                    if ((want[0] || want[1] || want[2] || want[3]) && give_up(spin, dead)) break;
+                    if ((want[0] || want[1] || want[2] || want[3]) && give_up(spin, dead, x.count, x.polls)) break;
                 }
             }
             __syncthreads();
@@ -941,6 +990,13 @@ __global__ __launch_bounds__(R2T) void k_sor_resident2(Resident2<T> x) {
         }
     }
 
+    if (!x.pl.whole) {
+        __syncthreads();
+        if (tid == 0) *dead = commit(x.count, x.target, *dead != 0, x.polls) ? 0 : 1;
+        __syncthreads();
+        if (*dead) return;
+    }
+
     // the owned rows and their periodic mirrors back to memory
     for (int e = tid; e < 2 * own * H; e += R2T) {
         const int lr = e / (2 * H), w = e - lr * (2 * H), c = w >= H, h = w - c * H, j = v0 + halo + lr;
@@ -952,8 +1008,6 @@ __global__ __launch_bounds__(R2T) void k_sor_resident2(Resident2<T> x) {
         if (j == 1) x.X[pf_soff(g, i, n + 1, 0)] = v;
     }
     wave_max_to_slot(err, x.slots);
-    __syncthreads();
-    if (tid == 0 && *dead) *x.fail = 1;
 }
 
 bool resident2_plan(const PfGeom &g, int bc, int iters, Resident2Plan &pl) {
@@ -997,15 +1051,15 @@ static hipError_t run_resident2(hipStream_t st, Resident2<T> &r) {
     const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     void *args[] = {&r};
-    if (r.pl.blocks == 1) return hipLaunchKernel(f, dim3(1), dim3(R2T), args, lds, st);
-    return hipLaunchCooperativeKernel(f, dim3((unsigned)r.pl.blocks), dim3(R2T), args, (unsigned)lds, st);
+    return hipLaunchKernel(f, dim3((unsigned)r.pl.blocks), dim3(R2T), args, lds, st);
 }
 
 template <typename T>
 hipError_t launch_resident2(hipStream_t st, const PfGeom &g, const StepArgs &a, const Resident2Plan &pl, int iters,
                             uint32_t seq, T *X, const T *R, const T *PHI, const double *phi, bool fast,
-                            unsigned long long *inbox, unsigned long long *slots, unsigned long long *fail) {
-    Resident2<T> r{g, a, pl, iters, seq, X, R, PHI, phi, inbox, slots, fail};
+                            unsigned long long *inbox, unsigned long long *slots, unsigned long long *count,
+                            unsigned long long target) {
+    Resident2<T> r{g, a, pl, iters, seq, X, R, PHI, phi, inbox, slots, count, target, resident_polls()};
 #define PF_R2(QQ)                                                                      \
     case QQ:                                                                           \
         return fast ? run_resident2<T, QQ, true>(st, r) : run_resident2<T, QQ, false>(st, r);
@@ -1021,9 +1075,11 @@ hipError_t launch_resident2(hipStream_t st, const PfGeom &g, const StepArgs &a, 
 }
 template hipError_t launch_resident2<double>(hipStream_t, const PfGeom &, const StepArgs &, const Resident2Plan &, int,
                                              uint32_t, double *, const double *, const double *, const double *, bool,
-                                             unsigned long long *, unsigned long long *, unsigned long long *);
+                                             unsigned long long *, unsigned long long *, unsigned long long *,
+                                            unsigned long long);
 template hipError_t launch_resident2<float>(hipStream_t, const PfGeom &, const StepArgs &, const Resident2Plan &, int,
                                             uint32_t, float *, const float *, const float *, const double *, bool,
-                                            unsigned long long *, unsigned long long *, unsigned long long *);
+                                            unsigned long long *, unsigned long long *, unsigned long long *,
+                                            unsigned long long);
 
 }  // namespace pf

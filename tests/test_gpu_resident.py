@@ -140,3 +140,57 @@ def _case_2d(size, iters, steps, step):
     some = rng.random(phi.shape) < 0.1
     phi[some] = rng.uniform(0.0, 1.0, int(some.sum()))
     return p, phi
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("dim", [2, 3])
+def test_a_launch_that_gives_up_leaves_the_solve_to_the_sweeps(dim, precision, monkeypatch):
+    """A wait of one poll: blocks give up, the launch changes nothing, and the context solves on
+    with the per-half-sweep kernels."""
+    from pixelflow_amd.solver import PF_PREC_FP64, PF_PREC_MIXED, Solver
+    p, phi = _case_2d((130, 40), 8, 3, False) if dim == 2 else _case("uniform", (64, 32, 32), 8, 3)
+    kw = dict(precision=PF_PREC_MIXED, inner_iters=8) if precision == "mixed" else dict(precision=PF_PREC_FP64)
+    fields = ("u", "v", "p") if dim == 2 else ("u", "v", "w", "p")
+    out = []
+    for polls in (None, "1"):
+        if polls:
+            monkeypatch.setenv("PF_RESIDENT_POLLS", polls)
+        monkeypatch.setenv("PF_RESIDENT", "1,2" if dim == 2 else "2,1,2")
+        with Solver(p, phi, **kw) as s:
+            assert s.sor_resident()
+            st = s.step(3)
+            assert s.sor_resident() == (polls is None)
+            out.append([s.interior(f) for f in fields] + [st["sor_error"]])
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
+
+
+def test_resident_contexts_in_two_threads():
+    """Two contexts, each of whose solves takes every CU, stepped from two threads at once."""
+    import threading
+
+    from pixelflow_amd.solver import Solver
+    p, phi = cases.sphere_case(m=256, n=128, l=128, steps=4, iter_max=10)
+    with Solver(p, phi) as s:
+        assert s.sor_resident()
+        s.step(4)
+        ref = s.interior("p")
+    out, errors = [None, None], []
+
+    def run(q):
+        try:
+            with Solver(p, phi) as s:
+                s.step(4)
+                out[q] = s.interior("p")
+        except Exception as e:   # reported by the main thread
+            errors.append(e)
+
+    print("[gpu] resident contexts in two threads", flush=True)
+    threads = [threading.Thread(target=run, args=(q,)) for q in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+    for x in out:
+        np.testing.assert_array_equal(x, ref)
