@@ -498,13 +498,19 @@ __global__ __launch_bounds__(RMAXT) void k_sor_resident(ResidentRun<T> r) {
     w.bb = (t.iz > 0 || periodic) ? at(t.ix, t.iy, t.iz > 0 ? t.iz - 1 : bz - 1) : -1;
     w.bt = (t.iz < bz - 1 || periodic) ? at(t.ix, t.iy, t.iz < bz - 1 ? t.iz + 1 : 0) : -1;
 
-    // the tile and its halo into LDS, the column's right-hand side into registers
+    // The tile and its halo into LDS, the column's right-hand side into registers.  Half-sweep 0
+    // takes periodic ghosts as they are in memory (an uploaded pressure's are what the caller
+    // gave), later ones the cells that they mirror.  Across an odd extent a ghost has its
+    // reader's colour: those that colour 1 reads are first read in half-sweep 1, before any
+    // message of that colour, so they come from their cells here.
+    const bool oddz = periodic && (r.g.l & 1);
     {
         const int wx = t.hx + 2, wxy = wx * (t.hy + 2), nc = wxy * t.hz;
         for (int e = tid; e < nc; e += nthr) {
             const int z = e / wxy, yx = e - z * wxy, yy = yx / wx, xx = yx - yy * wx;
-            const int ci = t.x0 - 1 + xx, cj = t.y0 - 1 + yy, ck = t.z0 + z;
-            L[(((ci + cj + ck) & 1) * NS + (z >> 1)) * RPL + yy * RP + xx] = r.X[pf_soff(r.g, ci, cj, ck)];
+            const int ci = t.x0 - 1 + xx, cj = t.y0 - 1 + yy, ck = t.z0 + z, par = (ci + cj + ck) & 1;
+            const int sj = (ODDY && par == 0) ? (cj == 0 ? r.g.n : cj == r.g.n + 1 ? 1 : cj) : cj;
+            L[(par * NS + (z >> 1)) * RPL + yy * RP + xx] = r.X[pf_soff(r.g, ci, sj, ck)];
         }
     }
     w.q0 = (i + j + t.z0) & 1;   // colour 1: 1 - q0
@@ -519,8 +525,10 @@ __global__ __launch_bounds__(RMAXT) void k_sor_resident(ResidentRun<T> r) {
             if (t.act && z < t.hz) w.b[c][s] = r.R[pf_soff(r.g, i, j, t.z0 + z)];
         }
     if (t.act) {
-        w.zlo = r.X[pf_soff(r.g, i, j, t.z0 - 1)];
-        w.zhi = r.X[pf_soff(r.g, i, j, t.z0 + t.hz)];
+        const bool lo = oddz && t.z0 == 1 && ((i + j + 1) & 1);
+        const bool hi = oddz && t.z0 + t.hz - 1 == r.g.l && ((i + j + r.g.l) & 1);
+        w.zlo = r.X[pf_soff(r.g, i, j, lo ? r.g.l : t.z0 - 1)];
+        w.zhi = r.X[pf_soff(r.g, i, j, hi ? 1 : t.z0 + t.hz)];
     }
     if constexpr (std::is_same<T, double>::value) {
         w.ce = w.cw = r.a.unit_ax;
