@@ -153,6 +153,22 @@ def build_serve_fake() -> str:
     return SERVE_FAKE
 
 
+HIP_STAND_IN = os.path.join(OUT, "test", "libhip_stand_in.so")
+
+
+def build_hip_stand_in() -> str:
+    """tests/native/hip_stand_in.cpp: the HIP calls of the library on host memory, for CPU
+    tests of its host code (which fail calls and look at what it does)."""
+    os.makedirs(os.path.dirname(HIP_STAND_IN), exist_ok=True)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    tmp = HIP_STAND_IN + ".tmp"
+    _run([shutil.which("g++") or "g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-Wno-deprecated-declarations",
+          "-D__HIP_PLATFORM_AMD__", f"-I{rocm}/include", os.path.join(ROOT, "tests", "native", "hip_stand_in.cpp"),
+          "-pthread", "-o", tmp])
+    os.replace(tmp, HIP_STAND_IN)
+    return HIP_STAND_IN
+
+
 def main(argv=None) -> int:
     ap = argparse.ArgumentParser()
     ap.add_argument("--lib-only", action="store_true")
@@ -163,6 +179,7 @@ def main(argv=None) -> int:
     if not args.lib_only:
         build_fortran()
         build_serve_fake()
+        build_hip_stand_in()
     if args.asan:
         build_asan_driver()
     return 0

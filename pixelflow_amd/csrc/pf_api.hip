@@ -669,18 +669,25 @@ extern "C" int pf_initial(pf_ctx *c) {
 // ------------------------------------------------------------------------------------
 // The time step
 // ------------------------------------------------------------------------------------
-// A solve of `iters` iterations as one resident launch; false where it does not apply.
-// What a resident launch of `blocks` blocks left: true with its result in place, false with
-// nothing changed (the half-sweep kernels take over).  Waits for the launch.
-static bool resident_done(pf_ctx *c, hipError_t e) {
-    if (e == hipSuccess) e = hipMemcpyAsync(c->rcount_host, c->rcount, 8, hipMemcpyDeviceToHost, c->st);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->st);
-    if (e == hipSuccess && *c->rcount_host == c->rtarget) return true;
-    (void)hipGetLastError();
-    // its blocks found no room beside other work on the GPU, or it could not be launched: this
-    // context stays with the half-sweep kernels
+// What enqueue_resident returns besides an error code (< 0, the step fails with it).
+enum { RESIDENT_NOT = 0, RESIDENT_DONE = 1 };
+
+// The outcome of a resident launch whose launch call returned `e`; waits for it.  Where blocks
+// gave up (they found no room beside other work on the GPU) or the launch was refused, nothing
+// has changed, the half-sweep kernels take over and this context stays with them.  If the count
+// cannot be read, the result may or may not be in place: the step fails.
+static int resident_done(pf_ctx *c, hipError_t e) {
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        c->resident = c->resident2 = false;
+        return RESIDENT_NOT;
+    }
+    PF_TRY_HIP(c, hipMemcpyAsync(c->rcount_host, c->rcount, 8, hipMemcpyDeviceToHost, c->st));
+    PF_TRY_HIP(c, hipStreamSynchronize(c->st));
+    if (*c->rcount_host == c->rtarget) return RESIDENT_DONE;
+    if (!(*c->rcount_host >> 63)) return fail(c, PF_EHIP, "a resident solve ended without an outcome");
     c->resident = c->resident2 = false;
-    return false;
+    return RESIDENT_NOT;
 }
 // Resident launches of this process, one at a time per device: two at once would keep each
 // other's last blocks out until both gave up.
@@ -689,11 +696,11 @@ static std::mutex &resident_lock(int device) {
     return locks[(unsigned)device % 16u];
 }
 
-static bool enqueue_resident2(pf_ctx *c, unsigned long long *slot, int iters) {
+static int enqueue_resident2(pf_ctx *c, unsigned long long *slot, int iters) {
     pf::Resident2Plan pl;
     if (!c->resident2 || c->fused || c->sor_variant == 0 || iters >= (1 << 28) ||
         !pf::resident2_plan(c->g, c->d.bc, iters, pl))
-        return false;
+        return RESIDENT_NOT;
     const bool f32 = c->d.precision == PF_PREC_MIXED, fast = c->sor_variant == 2;
     if (c->rseq > 0xffffffffu - (uint32_t)iters) {   // start over on an empty inbox
         pf::launch_clear_u64(c->st, c->rinbox, (int)pf::resident2_inbox_words(c->g, f32 ? 4 : 8));
@@ -710,15 +717,16 @@ static bool enqueue_resident2(pf_ctx *c, unsigned long long *slot, int iters) {
                                                             c->phi, fast, c->rinbox, slot, c->rcount, c->rtarget);
     c->rseq += (uint32_t)iters;
     if (!pl.whole) return resident_done(c, e);
-    if (e == hipSuccess) return true;   // one block waits for nobody
+    if (e == hipSuccess) return RESIDENT_DONE;   // one block waits for nobody
     (void)hipGetLastError();
     c->resident2 = false;
-    return false;
+    return RESIDENT_NOT;
 }
-static bool enqueue_resident(pf_ctx *c, unsigned long long *slot, int iters) {
+// A solve of `iters` iterations as one resident launch, where that applies.
+static int enqueue_resident(pf_ctx *c, unsigned long long *slot, int iters) {
     if (c->g.dim == 2) return enqueue_resident2(c, slot, iters);
     // the buffers' reuse needs messages of two iterations; the sequence numbers bound the count
-    if (!c->resident || !c->rcoef || c->fused || c->sor_variant == 0 || iters < 2 || iters >= (1 << 28)) return false;
+    if (!c->resident || !c->rcoef || c->fused || c->sor_variant == 0 || iters < 2 || iters >= (1 << 28)) return RESIDENT_NOT;
     const bool f32 = c->d.precision == PF_PREC_MIXED;
     if (c->rseq > 0xffffffffu - 2u * (uint32_t)iters) {   // start over on an empty inbox
         pf::launch_clear_u64(c->st, c->rinbox, (int)pf::resident_inbox_words(c->rpl, f32 ? 4 : 8));
@@ -735,7 +743,9 @@ static bool enqueue_resident(pf_ctx *c, unsigned long long *slot, int iters) {
     return resident_done(c, e);
 }
 
-static void enqueue_sor(pf_ctx *c, unsigned long long *slot, int iters) {
+static int enqueue_sor(pf_ctx *c, unsigned long long *slot, int iters) {
+    const int rc = enqueue_resident(c, slot, iters);
+    if (rc != RESIDENT_NOT) return rc < 0 ? rc : PF_OK;
     const PfGeom &g = c->g;
     const bool periodic = (c->d.bc == PF_BC_UNIFORM);
     const int fy = periodic && (g.n % 2 == 0);
@@ -745,7 +755,6 @@ static void enqueue_sor(pf_ctx *c, unsigned long long *slot, int iters) {
     // 3D sweeps (i+j+k) even first (:493), 2D sweeps (i+j) odd first (:339)
     const int first = (g.dim == 3) ? 0 : 1;
     int done = 0;
-    if (enqueue_resident(c, slot, iters)) return;
     if (c->tb2_k > 0 && c->sor_variant != 0 && iters >= 2) {
         // K iterations per launch, P -> P2 -> P ...: an even number of launches leaves the
         // result in P, so a launch of two or more iterations is split when the count is odd
@@ -804,6 +813,7 @@ static void enqueue_sor(pf_ctx *c, unsigned long long *slot, int iters) {
             if (ry || rz) pf::launch_ghost_refresh(c->st, g, ry, rz, c->P);
         }
     }
+    return PF_OK;
 }
 
 // Mixed precision pressure solve of one step (see pf_mixed.hip).  Returns cycles run;
@@ -856,7 +866,9 @@ static int enqueue_mixed(pf_ctx *c, unsigned long long *slot, double *res, int *
             if ((rc = residual(false)) != PF_OK) return rc;
         }
         const int kk = tol_mode ? K : (remaining < K ? remaining : K);
-        int done = enqueue_resident(c, slot, kk) ? kk : 0;
+        const int res_rc = enqueue_resident(c, slot, kk);
+        if (res_rc < 0) return res_rc;
+        int done = res_rc == RESIDENT_DONE ? kk : 0;
         if (c->fused && kk >= 2) {
             // E2's non-periodic ghosts are 0 like E's (zeroed at allocation, never written)
             for (; done + 2 <= kk; done += 2) {
@@ -932,7 +944,8 @@ static int enqueue_fp64_tol(pf_ctx *c, double *res, int *iters) {
         PF_TRY_HIP(c, hipStreamSynchronize(c->st));
         std::memcpy(res, &bits, sizeof(double));
         if (*res <= c->d.residual_tol || cyc == maxc || !std::isfinite(*res)) break;
-        enqueue_sor(c, c->err_part, K);
+        const int rc = enqueue_sor(c, c->err_part, K);
+        if (rc != PF_OK) return rc;
         *iters += K;
         ++cycles;
     }
@@ -987,7 +1000,8 @@ extern "C" int pf_step(pf_ctx *c, int nsteps, pf_stats *stats) {
             c->mixed_cycles.push_back(cyc);
             c->mixed_iters.push_back(iters);
         } else {
-            enqueue_sor(c, c->err_part, c->d.iter_max);
+            const int rc = enqueue_sor(c, c->err_part, c->d.iter_max);
+            if (rc != PF_OK) return rc;
         }
         if (c->mg32) pf::launch_reduce_err(c->st, c->mg32->err_slots, c->mg32->nslots, c->err + s);
         else if (c->mg64) pf::launch_reduce_err(c->st, c->mg64->err_slots, c->mg64->nslots, c->err + s);

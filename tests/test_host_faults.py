@@ -1,0 +1,87 @@
+"""What the host code does when a HIP call fails or a resident launch gives up, on the CPU:
+the library over a stand-in for the HIP runtime (tests/native/hip_stand_in.cpp) in a process
+of its own.  No kernel computes anything there; the tests look at error codes, at which
+kernels are launched, and at what is held afterwards."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+from pixelflow_amd import build, solver
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+pytestmark = pytest.mark.skipif(not os.path.exists(solver.LIB_PATH) or not os.path.exists(build.HIP_STAND_IN),
+                                reason="HIP library or its stand-in not built (python -m pixelflow_amd.build)")
+
+HEAD = """
+import ctypes, os, sys, threading
+import numpy as np
+from pixelflow_amd import build, cases, solver as S
+F = ctypes.CDLL(build.HIP_STAND_IN, mode=ctypes.RTLD_GLOBAL)   # before the library: its HIP calls go here
+F.fake_allocated.restype = ctypes.c_size_t
+F.fake_read.argtypes = [ctypes.c_void_p, ctypes.c_size_t]
+def launches(part): return F.fake_launches(part.encode())
+def fail(fn, skip=0, times=1, err=719): F.fake_fail(fn.encode(), skip, times, err)   # 719: hipErrorLaunchFailure
+def read(values, dtype="f8"):
+    a = np.asarray(values, dtype=dtype)
+    F.fake_read(a.ctypes.data, a.nbytes)
+def case(size=(64, 32, 32), iters=40):
+    m, n, l = size
+    p = cases.CaseParams(dim=3 if l > 1 else 2, m=m, n=n, l=l, width=0.01 * (m - 1), height=0.01 * (n - 1),
+                         depth=0.01 * (l - 1) if l > 1 else 0.0, time=1.0, istep_max=10**6, iter_max=iters)
+    return p, np.ones(p.interior_shape())
+def raises(f):
+    try: f()
+    except S.PixelFlowError as e: return str(e)
+    return None
+"""
+
+
+def run(body, **env):
+    r = subprocess.run([sys.executable, "-c", HEAD + textwrap.dedent(body) + "\nprint('ok')"], cwd=ROOT,
+                       env=dict(os.environ, **env), capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("where", ["count copy", "resident wait"])
+@pytest.mark.parametrize("kind", ["3d", "2d", "mixed", "tolerance"])
+def test_a_failed_wait_for_a_resident_solve_fails_the_step(where, kind):
+    """What the launch left is not known then: it may have written its result."""
+    run(f"""
+        kind, where = {kind!r}, {where!r}
+        p, phi = case((64, 32, 1) if kind == "2d" else (64, 32, 32))
+        if kind == "2d": os.environ["PF_RESIDENT"] = "1,2"
+        kw = dict(precision=S.PF_PREC_MIXED, inner_iters=20) if kind == "mixed" else {{}}
+        if kind == "tolerance":
+            kw = dict(residual_tol=1e-9)
+        with S.Solver(p, phi, **kw) as s:
+            assert s.sor_resident()
+            if kind == "tolerance": read([1.0])
+            s.step(1)
+            n = launches("k_sor_resident")
+            assert n >= 1
+            if kind == "tolerance": read([1.0])
+            fail(where)
+            msg = raises(lambda: s.step(1))
+            assert msg and "PF_EHIP" in msg, msg
+            assert launches("k_sor_resident") == n + 1
+            assert not launches("k_sor_phi") and not launches("k_sor32") and not launches("k_sor_tb2")
+    """)
+
+
+@pytest.mark.parametrize("kind", ["3d", "2d", "mixed"])
+def test_a_refused_launch_leaves_the_solve_to_the_sweeps(kind):
+    run(f"""
+        kind = {kind!r}
+        p, phi = case((64, 32, 1) if kind == "2d" else (64, 32, 32))
+        if kind == "2d": os.environ["PF_RESIDENT"] = "1,2"
+        kw = dict(precision=S.PF_PREC_MIXED, inner_iters=20) if kind == "mixed" else {{}}
+        with S.Solver(p, phi, **kw) as s:
+            fail("resident launch")
+            s.step(1)
+            assert not launches("k_sor_resident")
+            assert launches("k_sor_phi") + launches("k_sor32") + launches("k_sor_tb2")
+    """)
