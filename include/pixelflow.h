@@ -162,7 +162,9 @@ int pf_probe_copy(int64_t bytes, int iters, double *gbps);
  * colour-sweep launches (the default, faster on MI355X).  Same results. */
 int pf_sor_fused(const pf_ctx *ctx);
 /* 1 if the context solves a fixed count of SOR iterations as one launch that keeps the grid
- * on chip, 0 if with a launch per colour sweep or per few iterations.  Same results. */
+ * on chip, 0 if with a launch per colour sweep or per few iterations.  Same results.  The one
+ * launch needs room for all its blocks at once; where other processes' work leaves none it gives
+ * up, and the context pauses this form for 16 solves, then for longer, before it tries again. */
 int pf_sor_resident(const pf_ctx *ctx);
 /* 1 if the FP64 colour sweeps read the porosity coded in 4 bytes per value (values FP32
  * holds exactly as floats, the others through a table of at most 2^20 distinct doubles:

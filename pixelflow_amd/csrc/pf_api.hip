@@ -80,6 +80,8 @@ struct pf_ctx {
     unsigned long long *rcount = nullptr;  // blocks that finished, over all launches (device)
     unsigned long long *rcount_host = nullptr;   // pinned copy
     unsigned long long rtarget = 0;
+    int rpause = 0, rpaused = 0, rgood = 0;   // solves left of a pause after a launch that gave
+                                              // up, the pause's length, solves since
     pf::Downloader down;
     int err_cap = 0, nparts = 0;
     bool have_phi = false, have_init = false;
@@ -125,8 +127,8 @@ static bool desc_ok(const pf_desc *d, std::string &why) { return pf::desc_valid(
 extern "C" int pf_abi_version(void) { return PF_ABI_VERSION; }
 
 // The temporally blocked 2D sweep's iterations per launch and rows per block, or 0 and 0
-// where it is not used: FP64, 2D, and the shape within what the kernel holds, for contexts
-// whose solves are not resident (resident2_wanted).  By default 2
+// where it is not used: FP64, 2D, and the shape within what the kernel holds.  It also solves
+// for contexts of resident solves (resident2_wanted) while those pause.  By default 2
 // iterations and 1 row (on the 256x128 cylinder, ms per step: two-launch sweeps 0.86, K,R =
 // 1,1 0.60, 2,1 0.47, 2,2 0.54, 3,1 0.48, 4,1 0.52 with porosity in LDS, 4,8 0.80); rows
 // wider than about 310 cells do not fit LDS and keep the two-launch sweeps.
@@ -199,7 +201,7 @@ extern "C" int64_t pf_footprint_bytes(const pf_desc *d) {
         (d->precision == PF_PREC_FP64 && code_on) ? (int64_t)4 * 2 * g.HS + (int64_t)8 * PHI_TAB_MAX : 0;
     int tk = 0, tr = 0;
     const bool res2 = resident2_wanted(g, d);
-    if (!res2) tb2_params(g, d, tk, tr);
+    tb2_params(g, d, tk, tr);
     const int64_t p2 = (tk > 0) ? (int64_t)8 * 2 * g.HS : 0;
     const int64_t unit = unit_wanted(d) ? unit_flags_size(g) * (d->precision == PF_PREC_MIXED ? 2 : 1) : 0;
     pf::ResidentPlan pl;
@@ -336,7 +338,7 @@ extern "C" int pf_create(const pf_desc *desc, pf_ctx **out) {
         if (fv && *fv) c->fused = std::atoi(fv) != 0;
         c->fused = c->fused && pf::sor_fused_ok(g, desc->bc);
     }
-    if (!c->resident2) tb2_params(g, desc, c->tb2_k, c->tb2_r);
+    tb2_params(g, desc, c->tb2_k, c->tb2_r);
     if ((c->fused || c->tb2_k > 0) && desc->precision == PF_PREC_FP64 && (rc = alloc(c, &c->P2, 2 * g.HS)) != PF_OK)
         goto bad;
     if (desc->precision == PF_PREC_MIXED) {
@@ -673,9 +675,11 @@ extern "C" int pf_initial(pf_ctx *c) {
 enum { RESIDENT_NOT = 0, RESIDENT_DONE = 1 };
 
 // The outcome of a resident launch whose launch call returned `e`; waits for it.  Where blocks
-// gave up (they found no room beside other work on the GPU) or the launch was refused, nothing
-// has changed, the half-sweep kernels take over and this context stays with them.  If the count
-// cannot be read, the result may or may not be in place: the step fails.
+// gave up (they found no room beside other work on the GPU, which costs the wait of some 50 ms),
+// nothing has changed and the half-sweep kernels take over: for 16 solves, after each further
+// time for twice as many, up to 4096, until as many solves have gone well again.  A refused launch
+// is not tried again.  If the count cannot be read, the result may or may not be in place: the
+// step fails.
 static int resident_done(pf_ctx *c, hipError_t e) {
     if (e != hipSuccess) {
         (void)hipGetLastError();
@@ -684,9 +688,15 @@ static int resident_done(pf_ctx *c, hipError_t e) {
     }
     PF_TRY_HIP(c, hipMemcpyAsync(c->rcount_host, c->rcount, 8, hipMemcpyDeviceToHost, c->st));
     PF_TRY_HIP(c, hipStreamSynchronize(c->st));
-    if (*c->rcount_host == c->rtarget) return RESIDENT_DONE;
+    if (*c->rcount_host == c->rtarget) {
+        if (c->rpaused > 0 && ++c->rgood >= c->rpaused) c->rpaused = 0;
+        return RESIDENT_DONE;
+    }
     if (!(*c->rcount_host >> 63)) return fail(c, PF_EHIP, "a resident solve ended without an outcome");
-    c->resident = c->resident2 = false;
+    pf::launch_clear_u64(c->st, c->rcount, 1);
+    c->rtarget = 0;
+    c->rgood = 0;
+    c->rpause = c->rpaused = c->rpaused > 0 ? std::min(2 * c->rpaused, 4096) : 16;
     return RESIDENT_NOT;
 }
 // Resident launches of this process, one at a time per device: two at once would keep each
@@ -724,6 +734,10 @@ static int enqueue_resident2(pf_ctx *c, unsigned long long *slot, int iters) {
 }
 // A solve of `iters` iterations as one resident launch, where that applies.
 static int enqueue_resident(pf_ctx *c, unsigned long long *slot, int iters) {
+    if (c->rpause > 0) {
+        --c->rpause;
+        return RESIDENT_NOT;
+    }
     if (c->g.dim == 2) return enqueue_resident2(c, slot, iters);
     // the buffers' reuse needs messages of two iterations; the sequence numbers bound the count
     if (!c->resident || !c->rcoef || c->fused || c->sor_variant == 0 || iters < 2 || iters >= (1 << 28)) return RESIDENT_NOT;
@@ -1089,7 +1103,7 @@ extern "C" int pf_sor_fused(const pf_ctx *c) {
 
 extern "C" int pf_sor_resident(const pf_ctx *c) {
     if (!c) return PF_EINVAL;
-    if (c->fused || c->sor_variant == 0 || !c->have_phi) return 0;
+    if (c->fused || c->sor_variant == 0 || !c->have_phi || c->rpause > 0) return 0;
     return ((c->resident && c->rcoef) || c->resident2) ? 1 : 0;
 }
 

@@ -619,12 +619,14 @@ __global__ __launch_bounds__(RMAXT) void k_sor_resident(ResidentRun<T> r) {
 // ------------------------------------------------------------------------------------
 // Host side
 // ------------------------------------------------------------------------------------
-// Polls of a wait, at most: about 0.4 s of them.  PF_RESIDENT_POLLS in the environment sets
-// another number (tests: 1 makes launches give up).
+// Polls of a wait, at most: about 50 ms of them (a poll is a trip to memory, 0.8 us).  Blocks
+// that wait for others to be placed wait for the end of kernels in their way, a few ms; longer
+// than that is another process's resident launch that waits as well.  PF_RESIDENT_POLLS in the
+// environment sets another number (tests: 1 makes launches give up).
 static unsigned resident_polls() {
     const char *e = std::getenv("PF_RESIDENT_POLLS");
     const int v = (e && *e) ? std::atoi(e) : 0;
-    return v > 0 ? (unsigned)v : 1u << 19;
+    return v > 0 ? (unsigned)v : 1u << 16;
 }
 
 static int ns_of(int tz) {

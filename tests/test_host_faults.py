@@ -85,3 +85,30 @@ def test_a_refused_launch_leaves_the_solve_to_the_sweeps(kind):
             assert not launches("k_sor_resident")
             assert launches("k_sor_phi") + launches("k_sor32") + launches("k_sor_tb2")
     """)
+
+
+@pytest.mark.parametrize("kind", ["3d", "2d", "mixed"])
+def test_a_launch_that_gives_up_is_tried_again_after_a_pause(kind):
+    """16 solves by the sweeps (in 2D FP64 the blocked one), 32 after the next time,
+    and from then on resident again."""
+    run(f"""
+        kind = {kind!r}
+        p, phi = case((64, 32, 1) if kind == "2d" else (64, 32, 32))
+        if kind == "2d": os.environ["PF_RESIDENT"] = "1,2"
+        kw = dict(precision=S.PF_PREC_MIXED, inner_iters=40) if kind == "mixed" else {{}}
+        sweep = {{"3d": "k_sor_phi", "2d": "k_sor_tb2", "mixed": "k_sor32"}}[kind]
+        with S.Solver(p, phi, **kw) as s:
+            F.fake_give_up(2)
+            tries, solves = [], []
+            for step in range(80):
+                a, b = launches("k_sor_resident"), launches(sweep)
+                s.step(1)
+                if launches("k_sor_resident") > a: tries.append(step)
+                assert (launches(sweep) > b) == (step < 50), step   # 0..16 and 17..49
+                assert s.sor_resident() == (step in (16, 49) or step > 49), step
+            assert tries == [0, 17] + list(range(50, 80)), tries
+            F.fake_give_up(1)
+            for step in range(65):   # after 30 good solves of the 32 the pause doubles
+                s.step(1)
+            assert launches("k_sor_resident") == len(tries) + 1
+    """)
