@@ -40,6 +40,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 
@@ -634,6 +635,34 @@ static int ns_of(int tz) {
     return h <= 1 ? 1 : h <= 2 ? 2 : h <= 4 ? 4 : h <= 8 ? 8 : 16;
 }
 
+// Estimated us of a half-sweep for the slowest tile, one around a body: all of its waves read
+// coefficients.  A wave waits about 0.65 us a height pair for its seven loads, which other waves
+// of the SIMD cover until the CU's loads themselves take longer (0.074 us a wave and pair in FP64,
+// 0.034 in FP32); bottom and top messages cost by the tile's columns, more where they are not
+// packed (odd sides), side messages by a thread's share of them.  Fitted to 340 timings of 53
+// rooms, spheres and fields of boxes of 0.1 to 8 M cells with tilings of every shape; the
+// error is 4 to 5 % (rms).
+static double body_tile_us(const ResidentPlan &pl, int elem) {
+    const double pairs = (pl.tz + 1) / 2, waves = pl.threads / 64, columns = pl.tx * pl.ty;
+    const bool f64 = elem == 8, odd = ((pl.tx | pl.ty) & 1) != 0;
+    const double wait = 0.65 * pairs, loads = (f64 ? 0.074 : 0.034) * pairs * waves;
+    const double columns_us = f64 ? (odd ? 2.00e-3 : 1.66e-3) : (odd ? 0.93e-3 : 0.90e-3);
+    return (f64 ? 0.63 : 0.67) + std::pow(std::pow(wait, 4) + std::pow(loads, 4), 0.25) + columns_us * columns +
+           (f64 ? 0.42 : 0.24) * 2 * (pl.tx + pl.ty) * pairs / pl.threads;
+}
+// The same for a tile of unit cells: arithmetic of the fullest SIMD, and the surface.
+static double unit_tile_us(const ResidentPlan &pl) {
+    const int surface = 2 * ((pl.bx > 1 ? pl.ty : 0) + pl.tx) * pl.tz + 2 * pl.tx * pl.ty;
+    return (double)((pl.threads / 64 + 3) / 4) * ((pl.tz + 1) / 2) * 0.1 + surface * 0.0004;
+}
+
+// The tiling with the least body_tile_us, and of those within 3 % of it the one with the least
+// unit_tile_us: the slowest tile sets the pace of all.  By unit_tile_us alone a mixed room of
+// 105x113x87 got 15x17x22 tiles, eleven pairs in a row with nothing to cover their loads: 7.9 us a
+// half-sweep, streamed 6.4, now (27x29x6) 3.6.  us before / now: FP64 boxes 57x100x141 7.3 / 4.1,
+// sphere 139x117x46 7.3 / 3.8, room 160x128x96 8.3 / 7.3, sphere 256x128x128 unchanged; FP32 room
+// 128^3 6.7 / 4.6, 192x160x128 12.6 / 7.3, boxes 93x87x121 8.0 / 3.3; the worst of 53 grids, FP64
+// room 51x88x52, 2.53 / 2.59.
 bool resident_plan(const PfGeom &g, int elem, int cus, ResidentPlan &pl) {
     pl = ResidentPlan{};
     if (g.dim != 3 || g.m < 2 || g.n < 2 || g.l < 2) return false;
@@ -642,7 +671,8 @@ bool resident_plan(const PfGeom &g, int elem, int cus, ResidentPlan &pl) {
     int fx = 0, fy = 0, fz = 0;
     if (e && *e && std::sscanf(e, "%d,%d,%d", &fx, &fy, &fz) != 3) return false;
     const bool forced = fx > 0 && fy > 0 && fz > 0;
-    double best = 1e300;
+    double least = 1e300, unit = 1e300;
+    bool choosing = false;   // first pass: the least estimate; second: the choice
     auto consider = [&](int bx, int by, int bz) {
         const int tx = (g.m + bx - 1) / bx, ty = (g.n + by - 1) / by, tz = (g.l + bz - 1) / bz;
         if (tx > RT || ty > RT || tx * ty > RMAXT || (tz + 1) / 2 > maxns) return;
@@ -651,17 +681,21 @@ bool resident_plan(const PfGeom &g, int elem, int cus, ResidentPlan &pl) {
         bz = (g.l + tz - 1) / tz;
         if (bx * by * bz > cus) return;
         if (g.m - (bx - 1) * tx < 2 || g.n - (by - 1) * ty < 2) return;   // every tile two cells wide
-        const int ns = ns_of(tz), waves = (tx * ty + 63) / 64;
-        const int surface = 2 * ((bx > 1 ? ty : 0) + tx) * tz + 2 * tx * ty;
-        const double cost = (double)((waves + 3) / 4) * ((tz + 1) / 2) * 0.1 + surface * 0.0004;
-        if (cost < best) {
-            best = cost;
-            pl = ResidentPlan{bx, by, bz, tx, ty, tz, ns, waves * 64};
+        const ResidentPlan q{bx, by, bz, tx, ty, tz, ns_of(tz), (tx * ty + 63) / 64 * 64};
+        const double us = body_tile_us(q, elem);
+        if (!choosing) {
+            least = std::min(least, us);
+        } else if (us <= 1.03 * least && unit_tile_us(q) < unit) {
+            unit = unit_tile_us(q);
+            pl = q;
         }
     };
-    if (forced) {
-        consider(fx, fy, fz);
-    } else {
+    for (int pass = 0; pass < 2; ++pass) {
+        choosing = pass == 1;
+        if (forced) {
+            consider(fx, fy, fz);
+            continue;
+        }
         for (int bx = (g.m + RT - 1) / RT; bx <= cus && bx <= g.m; ++bx)
             for (int by = (g.n + RT - 1) / RT; bx * by <= cus && by <= g.n; ++by)
                 for (int bz = (g.l + 2 * maxns - 1) / (2 * maxns); bx * by * bz <= cus && bz <= g.l; ++bz)
