@@ -80,6 +80,7 @@ struct pf_ctx {
     unsigned long long *rcount = nullptr;  // blocks that finished, over all launches (device)
     unsigned long long *rcount_host = nullptr;   // pinned copy
     unsigned long long rtarget = 0;
+    int rmin = 2;                   // iterations of a resident solve, at least
     int rpause = 0, rpaused = 0, rgood = 0;   // solves left of a pause after a launch that gave
                                               // up, the pause's length, solves since
     pf::Downloader down;
@@ -152,8 +153,14 @@ static bool unit_wanted(const pf_desc *d) {
     return !(u && *u && std::atoi(u) == 0);
 }
 
-// Solves of a fixed SOR count run resident on chip where the grid fits (pf_resident.hip),
-// unless the environment selects a variant of the per-half-sweep kernels.
+// Iterations of a context's SOR solves (of a full cycle where it solves in cycles).
+static int solve_iters(const pf_desc *d) {
+    const bool cycles = d->precision == PF_PREC_MIXED || d->residual_tol > 0;
+    return cycles && d->inner_iters > 0 ? (d->residual_tol > 0 ? d->inner_iters : std::min(d->inner_iters, d->iter_max))
+                                        : d->iter_max;
+}
+// Solves of a fixed SOR count run resident on chip where the grid fits and they are long enough
+// (pf_resident.hip), unless the environment selects a variant of the per-half-sweep kernels.
 static bool resident_wanted(const PfGeom &g, const pf_desc *d, pf::ResidentPlan &pl) {
     if (g.dim != 3 || (d->residual_tol > 0 && d->solver == PF_SOLVER_MG)) return false;
     const char *own = std::getenv("PF_RESIDENT");
@@ -163,9 +170,10 @@ static bool resident_wanted(const PfGeom &g, const pf_desc *d, pf::ResidentPlan 
             const char *e = std::getenv(v);
             if (e && *e) return false;
         }
-    return pf::resident_plan(g, d->precision == PF_PREC_MIXED ? 4 : 8, pf::RESIDENT_CUS, pl);
+    const int elem = d->precision == PF_PREC_MIXED ? 4 : 8;
+    return solve_iters(d) >= pf::resident_min_iters(g, elem) && pf::resident_plan(g, elem, pf::RESIDENT_CUS, pl);
 }
-// The same in 2D (uniform inflow), and the plan for a solve of `iters` iterations.
+// The same in 2D (uniform inflow).
 static bool resident2_wanted(const PfGeom &g, const pf_desc *d) {
     pf::Resident2Plan pl;
     if (g.dim != 2 || (d->residual_tol > 0 && d->solver == PF_SOLVER_MG)) return false;
@@ -176,8 +184,9 @@ static bool resident2_wanted(const PfGeom &g, const pf_desc *d) {
             const char *e = std::getenv(v);
             if (e && *e) return false;
         }
-    const int iters = d->inner_iters > 0 && (d->precision == PF_PREC_MIXED || d->residual_tol > 0) ? d->inner_iters : d->iter_max;
-    return pf::resident2_plan(g, d->bc, std::max(2, iters), pl);
+    const int iters = solve_iters(d);
+    return pf::resident2_plan(g, d->bc, iters, pl) &&
+           (pl.whole || iters >= pf::resident_min_iters(g, d->precision == PF_PREC_MIXED ? 4 : 8));
 }
 static int64_t resident_bytes(const pf_desc *d, const pf::ResidentPlan &pl) {
     const int elem = d->precision == PF_PREC_MIXED ? 4 : 8;
@@ -293,6 +302,7 @@ extern "C" int pf_create(const pf_desc *desc, pf_ctx **out) {
     {
         int cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess) cus = 0;
+        c->rmin = pf::resident_min_iters(g, desc->precision == PF_PREC_MIXED ? 4 : 8);
         c->resident = resident_wanted(g, desc, c->rpl) && c->rpl.bx * c->rpl.by * c->rpl.bz <= cus;
         c->resident2 = resident2_wanted(g, desc) && cus >= pf::RESIDENT_CUS;
     }
@@ -709,7 +719,7 @@ static std::mutex &resident_lock(int device) {
 static int enqueue_resident2(pf_ctx *c, unsigned long long *slot, int iters) {
     pf::Resident2Plan pl;
     if (!c->resident2 || c->fused || c->sor_variant == 0 || iters >= (1 << 28) ||
-        !pf::resident2_plan(c->g, c->d.bc, iters, pl))
+        !pf::resident2_plan(c->g, c->d.bc, iters, pl) || (!pl.whole && iters < c->rmin))
         return RESIDENT_NOT;
     const bool f32 = c->d.precision == PF_PREC_MIXED, fast = c->sor_variant == 2;
     if (c->rseq > 0xffffffffu - (uint32_t)iters) {   // start over on an empty inbox
@@ -740,7 +750,8 @@ static int enqueue_resident(pf_ctx *c, unsigned long long *slot, int iters) {
     }
     if (c->g.dim == 2) return enqueue_resident2(c, slot, iters);
     // the buffers' reuse needs messages of two iterations; the sequence numbers bound the count
-    if (!c->resident || !c->rcoef || c->fused || c->sor_variant == 0 || iters < 2 || iters >= (1 << 28)) return RESIDENT_NOT;
+    if (!c->resident || !c->rcoef || c->fused || c->sor_variant == 0 || iters < c->rmin || iters >= (1 << 28))
+        return RESIDENT_NOT;
     const bool f32 = c->d.precision == PF_PREC_MIXED;
     if (c->rseq > 0xffffffffu - 2u * (uint32_t)iters) {   // start over on an empty inbox
         pf::launch_clear_u64(c->st, c->rinbox, (int)pf::resident_inbox_words(c->rpl, f32 ? 4 : 8));

@@ -119,6 +119,8 @@ constexpr int RESIDENT_CUS = 256;   // compute units of an MI355X: one workgroup
 // where the grid does not fit.  PF_RESIDENT="bx,by,bz" in the environment sets the tiles per
 // axis ("0": never).
 bool resident_plan(const PfGeom &g, int elem, int cus, ResidentPlan &pl);
+// Iterations that a solve needs to be one launch (but a 2D grid that one block holds: two).
+int resident_min_iters(const PfGeom &g, int elem);
 int64_t resident_inbox_words(const ResidentPlan &pl, int elem);
 // Waves of a launch, one error slot and one entry of `mask` and `first` each.
 int resident_waves(const ResidentPlan &pl);

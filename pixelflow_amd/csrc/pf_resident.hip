@@ -704,6 +704,23 @@ bool resident_plan(const PfGeom &g, int elem, int cus, ResidentPlan &pl) {
     return pl.bx > 0;
 }
 
+// The least iterations of a solve for which the one launch is faster.  It costs 30 to 80 us more
+// than sweeps do (the grid in and out of the chip, the agreement at the end, the host's wait for
+// it) and saves 4 to 15 us an iteration; us a step of 6 / 8 / 12 iterations, streamed and resident:
+// FP64 sphere 48x40x40 77, 77 / 92, 83 / 122, 96; room 64^3 107, 105 / 125, 114 / 160, 130; room 128^3
+// 317, 311 / 370, 339 / 477, 400; sphere 192x128x96 279, 290 / 321, 314 / 399, 363; FP32 sphere
+// 192x128x96 280, 302 / 309, 319 / 366, 354; 256x192x160 845, 868 / 910, 916 / 1036, 1011.  2D:
+// 256x128 51, 60 / 58, 64 / 76, 73; 768x384 78, 92 / 93, 102 / 124, 124; odd n, which the
+// sweeps follow with refreshes of the ghost rows, 511x255 93, 80 / 116, 88 / 165, 102.  A tiling
+// set in the environment is used for every solve of two or more.
+int resident_min_iters(const PfGeom &g, int elem) {
+    const char *e = std::getenv("PF_RESIDENT");
+    if (e && *e) return 2;
+    if (g.dim == 2) return (g.n & 1) ? 6 : 12;
+    if ((int64_t)g.m * g.n * g.l <= (1 << 19)) return 6;
+    return elem == 8 ? 8 : 12;
+}
+
 int resident_waves(const ResidentPlan &pl) { return pl.bx * pl.by * pl.bz * (pl.threads / 64); }
 int64_t resident_sets(const ResidentPlan &pl, const std::vector<uint32_t> &mask, std::vector<uint32_t> &first) {
     const uint32_t all = pl.ns == 16 ? 0xffffffffu : (1u << (2 * pl.ns)) - 1u;

@@ -1,6 +1,7 @@
-"""Resident solves by the rule's own choice of tiling give the bits of the oracle (FP64) and of
-the sweeps (mixed), at the edges of its ranges: the smallest grids, odd extents, sixteen FP32
-height pairs with a ragged last tile, rooms, and several cycles a step."""
+"""Which solves are resident by the rule's own choice, and that those that are give the bits of
+the oracle: tilings of the rule for both precisions at the edges of its ranges (the smallest
+grids, odd extents, sixteen FP32 height pairs with a ragged last tile, rooms), and iteration
+counts on either side of the least that it takes."""
 import numpy as np
 import pytest
 
@@ -74,3 +75,13 @@ def test_rule_mixed(kind, size, tiles, iters, monkeypatch):
             out.append([s.interior(f) for f in ("u", "v", "w", "p")] + [st["sor_error"]])
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("size,mixed,least", [((48, 40, 40), False, 6), ((48, 40, 40), True, 6), ((96, 96, 64), False, 8),
+                                              ((96, 96, 64), True, 12), ((130, 40, 1), False, 12), ((131, 41, 1), False, 6)])
+def test_short_solves_are_left_to_the_sweeps(size, mixed, least):
+    from pixelflow_amd.solver import PF_PREC_FP64, PF_PREC_MIXED, Solver
+    for iters in (least - 1, least):
+        p, phi = _case("uniform", size, iters, 1)
+        with Solver(p, phi, precision=PF_PREC_MIXED if mixed else PF_PREC_FP64) as s:
+            assert s.sor_resident() == (iters >= least)
