@@ -122,6 +122,8 @@ bool resident_plan(const PfGeom &g, int elem, int cus, ResidentPlan &pl);
 // Iterations that a solve needs to be one launch (but a 2D grid that one block holds: two).
 int resident_min_iters(const PfGeom &g, int elem);
 int64_t resident_inbox_words(const ResidentPlan &pl, int elem);
+// The quarters of a CU that a launch's blocks take.
+int resident_quarters(const ResidentPlan &pl, int elem);
 // Waves of a launch, one error slot and one entry of `mask` and `first` each.
 int resident_waves(const ResidentPlan &pl);
 // From the waves' masks: each wave's first coefficient set, and their count; a set is

@@ -736,6 +736,13 @@ int64_t resident_inbox_words(const ResidentPlan &pl, int elem) {
     return (int64_t)pl.bx * pl.by * pl.bz * 2 * (4 * 2 * pl.ns * RT + 2 * RMAXT) * (elem == 8 ? 2 : 1);
 }
 static size_t resident_lds(const ResidentPlan &pl, int elem) { return (size_t)2 * pl.ns * RPL * elem; }
+// The kernel's 1,024-thread bound leaves a wave 128 registers, a quarter of a SIMD's: a CU holds
+// sixteen waves, and blocks for as long as their LDS fits.
+int resident_quarters(const ResidentPlan &pl, int elem) {
+    const int by_waves = 16 / (pl.threads / 64), by_lds = (int)((size_t)(160 << 10) / (resident_lds(pl, elem) + 64));
+    const int per_cu = std::min(by_waves, by_lds);
+    return pl.bx * pl.by * pl.bz * (per_cu >= 4 ? 1 : per_cu >= 2 ? 2 : 4);
+}
 
 template <typename T, int NS, bool ODDY>
 static hipError_t run_resident(hipStream_t st, ResidentRun<T> &r) {

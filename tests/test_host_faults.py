@@ -112,3 +112,47 @@ def test_a_launch_that_gives_up_is_tried_again_after_a_pause(kind):
                 s.step(1)
             assert launches("k_sor_resident") == len(tries) + 1
     """)
+
+
+@pytest.mark.parametrize("tiles,together", [
+    ("2,1,2", 2),     # a few CUs each: both at once
+    ("8,4,8", 1),     # 256 blocks of a whole CU each: one after the other
+])
+def test_resident_launches_of_two_threads_share_the_chip(tiles, together):
+    run(f"""
+        os.environ["PF_RESIDENT"] = {tiles!r}
+        size = (64, 32, 32) if {together} == 2 else (256, 128, 128)
+        p, phi = case(size)
+        solvers = [S.Solver(p, phi) for _ in range(2)]
+        assert all(s.sor_resident() for s in solvers)
+        F.fake_hold(50)
+        threads = [threading.Thread(target=s.step, args=(3,)) for s in solvers]
+        for t in threads: t.start()
+        for t in threads: t.join()
+        assert F.fake_most_resident() == {together}, F.fake_most_resident()
+        assert launches("k_sor_resident") == 6 and not launches("k_sor_phi")
+    """)
+
+
+def test_resident_launches_take_turns_in_the_order_of_asking():
+    """A launch that needs the whole chip gets it although smaller ones keep coming."""
+    run("""
+        import time
+        os.environ["PF_RESIDENT"] = "2,1,2"
+        small = [S.Solver(*case((64, 32, 32))) for _ in range(3)]
+        os.environ["PF_RESIDENT"] = "8,4,8"
+        large = S.Solver(*case((256, 128, 128)))
+        F.fake_hold(20)
+        stop = threading.Event()
+        def keep(s):
+            while not stop.is_set(): s.step(1)
+        threads = [threading.Thread(target=keep, args=(s,)) for s in small]
+        for t in threads: t.start()
+        time.sleep(0.1)
+        t0 = time.perf_counter()
+        large.step(2)
+        took = time.perf_counter() - t0
+        stop.set()
+        for t in threads: t.join()
+        assert took < 5.0, took
+    """)
