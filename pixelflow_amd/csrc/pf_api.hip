@@ -232,6 +232,35 @@ static int alloc(pf_ctx *c, double **p, int64_t n) {
     return PF_OK;
 }
 
+static void resident_free(pf_ctx *c) {
+    void **all[] = {(void **)&c->rcoef, (void **)&c->rmask, (void **)&c->rfirst, (void **)&c->rinbox, (void **)&c->rcount};
+    for (void **p : all)
+        if (*p) { (void)hipFree(*p); *p = nullptr; }
+    c->rcoef_cap = 0;
+    if (c->rcount_host) { (void)hipHostFree(c->rcount_host); c->rcount_host = nullptr; }
+    c->resident = c->resident2 = false;
+}
+// What resident solves need besides the coefficients; a context without room for it solves by the
+// half-sweep kernels.
+static void resident_alloc(pf_ctx *c) {
+    if (!c->resident && !c->resident2) return;
+    const int elem = c->d.precision == PF_PREC_MIXED ? 4 : 8;
+    const int waves = c->resident ? pf::resident_waves(c->rpl) : pf::RESIDENT_CUS * 8;
+    const int64_t words = c->resident ? pf::resident_inbox_words(c->rpl, elem) : pf::resident2_inbox_words(c->g, elem);
+    if (hipMalloc((void **)&c->rcount, 8) != hipSuccess ||
+        hipHostMalloc((void **)&c->rcount_host, 8, hipHostMallocDefault) != hipSuccess ||
+        hipMalloc((void **)&c->rinbox, (size_t)words * 8) != hipSuccess ||
+        (c->resident && (hipMalloc((void **)&c->rmask, (size_t)waves * 4) != hipSuccess ||
+                         hipMalloc((void **)&c->rfirst, (size_t)waves * 4) != hipSuccess))) {
+        (void)hipGetLastError();
+        resident_free(c);
+        return;
+    }
+    c->nparts = std::max(c->nparts, waves);
+    pf::launch_clear_u64(c->st, c->rcount, 1);
+    pf::launch_clear_u64(c->st, c->rinbox, (int)words);
+}
+
 static void release(pf_ctx *c) {
     double **all[] = {&c->u, &c->v, &c->w, &c->uo, &c->vo, &c->wo, &c->phi, &c->div, &c->dout,
                       &c->P, &c->BB, &c->AW, &c->AS, &c->AB, &c->PHIs, &c->force_buf, &c->P2};
@@ -247,12 +276,7 @@ static void release(pf_ctx *c) {
     if (c->PHTAB) { (void)hipFree(c->PHTAB); c->PHTAB = nullptr; }
     if (c->UNIT) { (void)hipFree(c->UNIT); c->UNIT = nullptr; }
     if (c->UNIT32) { (void)hipFree(c->UNIT32); c->UNIT32 = nullptr; }
-    if (c->rcoef) { (void)hipFree(c->rcoef); c->rcoef = nullptr; }
-    if (c->rmask) { (void)hipFree(c->rmask); c->rmask = nullptr; }
-    if (c->rfirst) { (void)hipFree(c->rfirst); c->rfirst = nullptr; }
-    if (c->rinbox) { (void)hipFree(c->rinbox); c->rinbox = nullptr; }
-    if (c->rcount) { (void)hipFree(c->rcount); c->rcount = nullptr; }
-    if (c->rcount_host) { (void)hipHostFree(c->rcount_host); c->rcount_host = nullptr; }
+    resident_free(c);
     if (c->mg32) { pf::mg_destroy(*c->mg32); delete c->mg32; c->mg32 = nullptr; }
     if (c->mg64) { pf::mg_destroy(*c->mg64); delete c->mg64; c->mg64 = nullptr; }
     for (hipEvent_t e : c->evs) (void)hipEventDestroy(e);
@@ -308,35 +332,7 @@ extern "C" int pf_create(const pf_desc *desc, pf_ctx **out) {
         c->resident = resident_wanted(g, desc, c->rpl) && c->rpl.bx * c->rpl.by * c->rpl.bz <= cus;
         c->resident2 = resident2_wanted(g, desc) && cus >= pf::RESIDENT_CUS;
     }
-    if (c->resident || c->resident2) {
-        if (hipMalloc((void **)&c->rcount, 8) != hipSuccess ||
-            hipHostMalloc((void **)&c->rcount_host, 8, hipHostMallocDefault) != hipSuccess) {
-            rc = fail(c, PF_ENOMEM, "hipMalloc of the resident sweep's count failed");
-            goto bad;
-        }
-        pf::launch_clear_u64(c->st, c->rcount, 1);
-    }
-    if (c->resident2) {
-        const int64_t words = pf::resident2_inbox_words(g, desc->precision == PF_PREC_MIXED ? 4 : 8);
-        c->nparts = std::max(c->nparts, pf::RESIDENT_CUS * 8);
-        if (hipMalloc((void **)&c->rinbox, (size_t)words * 8) != hipSuccess) {
-            rc = fail(c, PF_ENOMEM, "hipMalloc of the resident sweep's arrays failed");
-            goto bad;
-        }
-        pf::launch_clear_u64(c->st, c->rinbox, (int)words);
-    }
-    if (c->resident) {
-        const int nw = pf::resident_waves(c->rpl);
-        const int64_t words = pf::resident_inbox_words(c->rpl, desc->precision == PF_PREC_MIXED ? 4 : 8);
-        c->nparts = std::max(c->nparts, nw);
-        if (hipMalloc((void **)&c->rmask, (size_t)nw * 4) != hipSuccess ||
-            hipMalloc((void **)&c->rfirst, (size_t)nw * 4) != hipSuccess ||
-            hipMalloc((void **)&c->rinbox, (size_t)words * 8) != hipSuccess) {
-            rc = fail(c, PF_ENOMEM, "hipMalloc of the resident sweep's arrays failed");
-            goto bad;
-        }
-        pf::launch_clear_u64(c->st, c->rinbox, (int)words);
-    }
+    resident_alloc(c);
     if (hipMalloc((void **)&c->err_part, sizeof(unsigned long long) * (size_t)c->nparts) != hipSuccess ||
         hipMalloc((void **)&c->res_part, sizeof(unsigned long long) * (size_t)c->nparts) != hipSuccess ||
         hipMalloc((void **)&c->res_val, sizeof(unsigned long long)) != hipSuccess) {

@@ -22,6 +22,7 @@ std::mutex g_mu;
 thread_local hipError_t t_last = hipSuccess;
 struct Fault { int skip, times; hipError_t err; };
 std::map<std::string, Fault> g_faults;
+std::map<std::string, int> g_calls;
 std::map<const void *, std::string> g_kernels;
 std::vector<std::string> g_log;
 std::map<size_t, std::deque<std::vector<char>>> g_reads;   // by size: what later device-to-host copies deliver
@@ -38,6 +39,7 @@ hipError_t done(hipError_t e) {
 }
 // The scripted error of a call, if it is its turn.
 hipError_t scripted(const char *fn) {
+    ++g_calls[fn];
     auto it = g_faults.find(fn);
     if (it == g_faults.end()) return hipSuccess;
     Fault &f = it->second;
@@ -63,6 +65,7 @@ extern "C" {
 void fake_reset() {
     std::lock_guard<std::mutex> lk(g_mu);
     g_faults.clear();
+    g_calls.clear();
     g_log.clear();
     g_reads.clear();
     g_give_up = g_hold_ms = g_most = 0;
@@ -90,6 +93,7 @@ int fake_launches(const char *part) {
     for (const auto &s : g_log) n += s.find(part) != std::string::npos;
     return n;
 }
+int fake_calls(const char *fn) { return g_calls[fn]; }
 int fake_most_resident() { return g_most; }
 unsigned fake_most_resident_blocks() { return g_most_blocks; }
 size_t fake_allocated() { return g_allocated; }

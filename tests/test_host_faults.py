@@ -25,6 +25,7 @@ F.fake_allocated.restype = ctypes.c_size_t
 F.fake_read.argtypes = [ctypes.c_void_p, ctypes.c_size_t]
 def launches(part): return F.fake_launches(part.encode())
 def fail(fn, skip=0, times=1, err=719): F.fake_fail(fn.encode(), skip, times, err)   # 719: hipErrorLaunchFailure
+def calls(fn): return F.fake_calls(fn.encode())
 def read(values, dtype="f8"):
     a = np.asarray(values, dtype=dtype)
     F.fake_read(a.ctypes.data, a.nbytes)
@@ -155,4 +156,45 @@ def test_resident_launches_take_turns_in_the_order_of_asking():
         stop.set()
         for t in threads: t.join()
         assert took < 5.0, took
+    """)
+
+
+@pytest.mark.parametrize("kind", ["3d", "2d", "mixed"])
+def test_no_room_for_the_resident_form_leaves_the_sweeps(kind):
+    """Each allocation of pf_create fails once: those of the resident form leave a context that
+    solves by the sweeps, any other fails the call; nothing is left behind."""
+    run(f"""
+        kind = {kind!r}
+        p, phi = case((130, 40, 1) if kind == "2d" else (64, 32, 32))
+        kw = dict(precision=S.PF_PREC_MIXED, inner_iters=20) if kind == "mixed" else {{}}
+        def mallocs(mode):
+            os.environ["PF_RESIDENT"] = mode
+            F.fake_reset()
+            S.Solver(p, phi, **kw).close()
+            os.environ.pop("PF_RESIDENT")
+            return calls("hipMalloc")
+        own = mallocs("") - mallocs("0")
+        own -= 1 if kind != "2d" else 0      # the coefficients, of pf_set_porosity
+        assert own == (2 if kind == "2d" else 4), own
+        n, sweeps = mallocs(""), 0
+        for at in range(n):
+            F.fake_reset()
+            fail("hipMalloc", skip=at, err=2)   # hipErrorOutOfMemory
+            try:
+                s = S.Solver(p, phi, **kw)
+            except S.PixelFlowError as e:
+                assert "PF_ENOMEM" in str(e) or "PF_EHIP" in str(e), e
+            else:
+                sweeps += not s.sor_resident()
+                s.step(2)
+                assert bool(launches("k_sor_resident")) == s.sor_resident()
+                s.close()
+            assert F.fake_allocated() == 0, at
+        assert sweeps == own + (kind != "2d"), sweeps
+        F.fake_reset()
+        fail("hipHostMalloc", err=2)
+        with S.Solver(p, phi, **kw) as s:
+            assert not s.sor_resident()
+            s.step(2)
+        assert F.fake_allocated() == 0
     """)
