@@ -76,6 +76,7 @@ struct pf_ctx {
     pf::ResidentPlan rpl{};
     void *rcoef = nullptr;          // double or float by precision, sized by the porosity
     size_t rcoef_cap = 0;
+    bool rready = false;            // masks and coefficients are the current porosity's
     uint32_t *rmask = nullptr, *rfirst = nullptr;
     unsigned long long *rinbox = nullptr;
     uint32_t rseq = 1;              // next unused message sequence number
@@ -509,6 +510,7 @@ static int resident_from_porosity(pf_ctx *c) {
     PF_TRY_HIP(c, hipMemcpyAsync(c->rfirst, first.data(), first.size() * 4, hipMemcpyHostToDevice, c->st));
     setup(c->rfirst);
     PF_TRY_HIP(c, hipStreamSynchronize(c->st));   // `first` is on this stack frame
+    c->rready = true;
     return PF_OK;
 }
 
@@ -516,6 +518,7 @@ static int resident_from_porosity(pf_ctx *c) {
 // the choice of sweep kernel.
 static int derive_from_porosity(pf_ctx *c) {
     const PfGeom &g = c->g;
+    c->rready = false;
     pf::launch_faces(c->st, g, c->phi, c->AW, c->AS, c->AB, c->d.dt, c->d.dx, c->d.dy, g.dim == 3 ? c->d.dz : 1.0);
     pf::launch_split(c->st, g, c->phi, c->PHIs);
     if (c->PHI32) pf::launch_split32(c->st, g, c->phi, c->PHI32);
@@ -593,6 +596,7 @@ extern "C" int pf_set_porosity(pf_ctx *c, const double *raw, double threshold) {
     if (!c || !raw) return PF_EINVAL;
     std::vector<double> phi;
     pf::host_porosity(c->g, c->d.bc, raw, threshold, phi);
+    c->rready = false;
     PF_TRY_HIP(c, hipMemcpyAsync(c->phi, phi.data(), phi.size() * sizeof(double), hipMemcpyHostToDevice, c->st));
     return derive_from_porosity(c);
 }
@@ -790,7 +794,7 @@ static int enqueue_resident(pf_ctx *c, unsigned long long *slot, int iters) {
     }
     if (c->g.dim == 2) return enqueue_resident2(c, slot, iters);
     // the buffers' reuse needs messages of two iterations; the sequence numbers bound the count
-    if (!c->resident || !c->rcoef || c->fused || c->sor_variant == 0 || iters < c->rmin || iters >= (1 << 28))
+    if (!c->resident || !c->rready || c->fused || c->sor_variant == 0 || iters < c->rmin || iters >= (1 << 28))
         return RESIDENT_NOT;
     const bool f32 = c->d.precision == PF_PREC_MIXED;
     if (c->rseq > 0xffffffffu - 2u * (uint32_t)iters) {   // start over on an empty inbox
@@ -1155,7 +1159,7 @@ extern "C" int pf_sor_fused(const pf_ctx *c) {
 extern "C" int pf_sor_resident(const pf_ctx *c) {
     if (!c) return PF_EINVAL;
     if (c->fused || c->sor_variant == 0 || !c->have_phi || c->rpause > 0) return 0;
-    return ((c->resident && c->rcoef) || c->resident2) ? 1 : 0;
+    return ((c->resident && c->rready) || c->resident2) ? 1 : 0;
 }
 
 extern "C" int pf_set_timing(pf_ctx *c, int on) {

@@ -198,3 +198,34 @@ def test_no_room_for_the_resident_form_leaves_the_sweeps(kind):
             s.step(2)
         assert F.fake_allocated() == 0
     """)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_a_porosity_that_was_not_set_up_is_not_solved_resident(precision):
+    """pf_set_porosity fails before the masks and coefficients are those of one porosity: a later
+    step does not launch on them; with a porosity that was set up it does again."""
+    run(f"""
+        kw = dict(precision=S.PF_PREC_MIXED, inner_iters=20) if {precision!r} == "mixed" else {{}}
+        p, phi = case()
+        raw = np.random.default_rng(1).random(phi.size)
+        failed = 0
+        for fn in ("hipMemcpyAsync", "hipStreamSynchronize"):
+            for at in range(12):
+                F.fake_reset()
+                with S.Solver(p, phi, **kw) as s:
+                    s.step(1)
+                    assert s.sor_resident() and launches("k_sor_resident")
+                    F.fake_reset()
+                    fail(fn, skip=at)
+                    rc = S.lib().pf_set_porosity(s._h, S._dp(raw), float(p.threshold))
+                    if rc == 0 or launches("k_resident_setup") > 1: continue   # none failed, or a later one
+                    failed += 1
+                    F.fake_reset()
+                    assert not s.sor_resident(), (fn, at)
+                    s.step(1)
+                    assert not launches("k_sor_resident"), (fn, at)
+                    s._check(S.lib().pf_set_porosity(s._h, S._dp(raw), float(p.threshold)), "pf_set_porosity")
+                    s.step(1)
+                    assert s.sor_resident() and launches("k_sor_resident")
+        assert failed >= 6, failed
+    """)
