@@ -1697,7 +1697,15 @@ static bool iteration_graph(MgSolver<T> &S, hipStream_t st) {
 // boundary, which a graph does not shorten, and keeps its launches.
 template <typename T>
 static void enqueue_iteration(MgSolver<T> &S, hipStream_t st, bool shared) {
-    if (!(shared && iteration_graph(S, st) && hipGraphLaunch(S.gexec, st) == hipSuccess)) launch_iteration(S, st);
+    bool launched = shared && iteration_graph(S, st);
+    if (launched && hipGraphLaunch(S.gexec, st) != hipSuccess) {
+        // refused, so nothing of it runs: the kernels one by one from now on
+        (void)hipGetLastError();
+        drop_graph(S);
+        S.graph_failed = true;
+        launched = false;
+    }
+    if (!launched) launch_iteration(S, st);
     (void)hipMemcpyAsync(S.h_scal, S.scal, 8 * sizeof(double), hipMemcpyDeviceToHost, st);
     S.vcycles += 2;
 }

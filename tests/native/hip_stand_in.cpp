@@ -26,7 +26,8 @@ std::map<std::string, int> g_calls;
 std::map<const void *, std::string> g_kernels;
 std::vector<std::string> g_log;
 std::map<size_t, std::deque<std::vector<char>>> g_reads;   // by size: what later device-to-host copies deliver
-struct Stream { int pending = 0; unsigned blocks = 0; };    // resident launches not yet waited for
+// pending: a resident launch not yet waited for
+struct Stream { int pending = 0; unsigned blocks = 0; bool capturing = false; };
 int g_give_up = 0, g_hold_ms = 0;
 unsigned g_blocks = 0, g_most_blocks = 0;
 int g_inflight = 0, g_most = 0;
@@ -120,6 +121,7 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *s, hipStream_t *s
 }
 hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **args, size_t, hipStream_t st) {
     CALL("hipLaunchKernel");
+    if (st && ((Stream *)st)->capturing) return hipSuccess;
     const std::string &name = g_kernels[f];
     const bool resident = name.find("k_sor_resident") != std::string::npos;
     if (resident) {
@@ -261,8 +263,13 @@ hipError_t hipEventDestroy(hipEvent_t e) { delete (int *)e; return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { CALL("hipEventRecord"); return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { CALL("hipEventSynchronize"); return hipSuccess; }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { *ms = 1.f; return hipSuccess; }
-hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { CALL("hipStreamBeginCapture"); return hipSuccess; }
-hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) {
+hipError_t hipStreamBeginCapture(hipStream_t st, hipStreamCaptureMode) {
+    CALL("hipStreamBeginCapture");
+    ((Stream *)st)->capturing = true;
+    return hipSuccess;
+}
+hipError_t hipStreamEndCapture(hipStream_t st, hipGraph_t *g) {
+    ((Stream *)st)->capturing = false;
     CALL("hipStreamEndCapture");
     *g = (hipGraph_t) new int(0);
     return hipSuccess;

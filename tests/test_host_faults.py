@@ -229,3 +229,35 @@ def test_a_porosity_that_was_not_set_up_is_not_solved_resident(precision):
                     assert s.sor_resident() and launches("k_sor_resident")
         assert failed >= 6, failed
     """)
+
+
+@pytest.mark.parametrize("call", ["hipGraphLaunch", "hipGraphInstantiate", "hipStreamBeginCapture", "hipStreamEndCapture"])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_a_graph_that_fails_leaves_the_iteration_to_launches(call, precision):
+    """A batch's multigrid solves launch an iteration as one graph; where that fails the kernels
+    are launched one by one, the step succeeds and the graph is not tried again."""
+    run(f"""
+        kw = dict(residual_tol=1e-9, solver=S.PF_SOLVER_MG, max_cycles=30)
+        if {precision!r} == "mixed": kw["precision"] = S.PF_PREC_MIXED
+        p, phi = case((16, 16, 16))
+        arena = 2 * S.batch_case_bytes(p, **kw) + (64 << 20)
+        b = S.Batch(p, max_cases=2, arena_bytes=arena, **kw)
+        for _ in range(2): b.add(p, phi)
+        def step():   # residual 1, an inner solve that ends after one iteration, residual 0; per case
+            for v in (1.0, 1.0, 0.0, 0.0): read([v])
+            for _ in range(2): read([0, 0, 0, 0, 1.0, 1.0, 0, 0])
+            for _ in range(2): read([0, 0, 0, 0, 1.0, 0.0, 0, 0])
+            b.step(1)
+        step()
+        assert launches("graph") == 2, launches("graph")
+        b.close()
+        F.fake_reset()
+        b = S.Batch(p, max_cases=2, arena_bytes=arena, **kw)
+        for _ in range(2): b.add(p, phi)
+        fail({call!r}, times=2)
+        step()
+        assert not launches("graph") and launches("k_bicg_xr") == 2, (launches("graph"), launches("k_bicg_xr"))
+        step()
+        assert not launches("graph") and launches("k_bicg_xr") == 4
+        b.close()
+    """)
