@@ -104,9 +104,28 @@ hipError_t Downloader::reserve(size_t bytes, int buffers) {
         e = hipHostMalloc(&pin[b], std::max(bytes, cap), hipHostMallocDefault);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&done[b], hipEventDisableTiming);
     }
-    if (e != hipSuccess) release();
-    else cap = std::max(bytes, cap);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        release();
+    } else {
+        cap = std::max(bytes, cap);
+    }
     return e;
+}
+
+// Without pinned memory: the device layout as it is, put in order here.
+static hipError_t get_staged(hipStream_t st, const PfGeom &g, bool split, const double *src, double *host, int64_t ldi,
+                             int64_t ldj) {
+    std::vector<double> stage((size_t)(split ? 2 * g.HS : g.NS));
+    hipError_t e = hipStreamSynchronize(st);
+    if (e == hipSuccess) e = hipMemcpy(stage.data(), src, stage.size() * sizeof(double), hipMemcpyDeviceToHost);
+    if (e != hipSuccess) return e;
+    for (int k = 0; k < g.Z; ++k)
+        for (int j = 0; j < g.Y; ++j)
+            for (int i = 0; i < g.m + 2; ++i)
+                host[(size_t)i + (size_t)ldi * ((size_t)j + (size_t)ldj * (size_t)k)] =
+                    stage[(size_t)(split ? pf_soff(g, i, j, k) : pf_off(g, i, j, k))];
+    return hipSuccess;
 }
 
 hipError_t Downloader::get(hipStream_t st, const PfGeom &g, bool split, const double *src, double *host, int64_t ldi,
@@ -130,7 +149,7 @@ hipError_t Downloader::chunks(hipStream_t st, const PfGeom &g, bool split, const
     const int per = (int)std::max<size_t>(1, std::min<size_t>((size_t)rows, CHUNK / row));
     const int n = (rows + per - 1) / per;
     hipError_t e = reserve(((size_t)per * row + 15) / 16 * 16, n > 1 ? 2 : 1);
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess) return get_staged(st, g, split, src, host, ldi, ldj);
     const int cpus = (size_t)per * row >= 2 * PER_THREAD ? cpu_share() : 1;
     auto send = [&](int c) -> hipError_t {
         const int row0 = c * per;

@@ -1,10 +1,12 @@
 // A stand-in for the HIP runtime on host memory, for CPU tests of the library's host code
 // (tests/test_host_faults.py loads it before libpixelflow.so, whose HIP calls then come here).
-// Device memory is host memory; kernels do nothing, except that k_clear_u64 clears and a
-// resident sweep's launch counts its blocks in (or leaves the give-up bit).  Any call can be
+// Device memory is host memory; kernels do nothing, except that k_clear_u64 clears, k_pack fills
+// the rows with its source's first value that is not 0, and a resident sweep's launch counts its
+// blocks in (or leaves the give-up bit).  Any call can be
 // made to fail, and what the host reads back can be set.
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
@@ -80,7 +82,7 @@ void fake_fail(const char *fn, int skip, int times, int err) {
 }
 // The next `n` resident launches give up.
 void fake_give_up(int n) { g_give_up = n; }
-// A wait for a stream that holds a resident launch takes this long.
+// A wait for an event, or for a stream that holds a resident launch, takes this long.
 void fake_hold(int ms) { g_hold_ms = ms; }
 // The next device-to-host copy of `bytes` bytes delivers `data` (a queue per size).
 void fake_read(const void *data, size_t bytes) {
@@ -136,6 +138,11 @@ hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **args, size_t, 
     }
     if (name.find("k_clear_u64") != std::string::npos)
         std::memset(*(void **)args[0], 0, (size_t) * (int *)args[1] * 8);
+    if (name.find("k_pack") != std::string::npos) {
+        const double *src = *(const double **)args[1];
+        while (*src == 0.) ++src;
+        std::fill_n(*(double **)args[2], *(unsigned *)args[4], *src);
+    }
     g_log.push_back(name);
     return hipSuccess;
 }
@@ -261,7 +268,11 @@ hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
 }
 hipError_t hipEventDestroy(hipEvent_t e) { delete (int *)e; return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { CALL("hipEventRecord"); return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { CALL("hipEventSynchronize"); return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) {
+    if (g_hold_ms) std::this_thread::sleep_for(std::chrono::milliseconds(g_hold_ms));
+    CALL("hipEventSynchronize");
+    return hipSuccess;
+}
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { *ms = 1.f; return hipSuccess; }
 hipError_t hipStreamBeginCapture(hipStream_t st, hipStreamCaptureMode) {
     CALL("hipStreamBeginCapture");

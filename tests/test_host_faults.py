@@ -261,3 +261,29 @@ def test_a_graph_that_fails_leaves_the_iteration_to_launches(call, precision):
         assert not launches("graph") and launches("k_bicg_xr") == 4
         b.close()
     """)
+
+
+@pytest.mark.parametrize("call", ["hipHostMalloc", "hipEventCreateWithFlags"])
+@pytest.mark.parametrize("dim", [2, 3])
+def test_fields_come_without_pinned_memory(call, dim):
+    run(f"""
+        os.environ["PF_RESIDENT"] = "0"
+        p, phi = case((33, 21, 1) if {dim} == 2 else (33, 21, 13))
+        rng = np.random.default_rng(2)
+        s = S.Solver(p, phi)
+        b = S.Batch(p, max_cases=1, arena_bytes=S.batch_case_bytes(p) + (64 << 20))
+        slot = b.add(p, phi)
+        fail({call!r}, times=-1)
+        for f in ("u", "v", "p"):
+            a = rng.standard_normal(p.full_shape())
+            s.set_field(f, a)
+            np.testing.assert_array_equal(s.field(f), a)
+            assert b.field(slot, f).shape == p.full_shape()
+            assert F.hipGetLastError() == 0
+        assert not launches("k_pack")
+        ldi, ldj = p.m + 5, p.n + 3
+        wide = np.full((p.l + 2 if {dim} == 3 else 1, ldj, ldi), -7.0)
+        assert S.lib().pf_download(s._h, S.FIELDS["p"], S._dp(wide), ldi, ldj) == 0
+        np.testing.assert_array_equal(wide[:, :p.n + 2, :p.m + 2].reshape(p.full_shape()), a)
+        assert (wide[:, p.n + 2:, :] == -7.0).all() and (wide[:, :, p.m + 2:] == -7.0).all()
+    """)
