@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
+#include <mutex>
+
 #include "pf_layout.h"
 
 namespace pf {
@@ -15,11 +17,13 @@ struct Downloader {
     size_t cap = 0;
     // The field src (colour-split or natural layout) after all work queued on st, into host
     // storage with leading dimensions ldi >= m + 2 and ldj >= n + 2; returns when it is there.
+    // Calls of several threads take turns.
     hipError_t get(hipStream_t st, const PfGeom &g, bool split, const double *src, double *host, int64_t ldi,
                    int64_t ldj);
     void release();
 
    private:
+    std::mutex turn;   // of the buffers
     hipError_t reserve(size_t bytes, int buffers);
     hipError_t chunks(hipStream_t st, const PfGeom &g, bool split, const double *src, double *host, int64_t ldi,
                       int64_t ldj);

@@ -130,6 +130,7 @@ static hipError_t get_staged(hipStream_t st, const PfGeom &g, bool split, const 
 
 hipError_t Downloader::get(hipStream_t st, const PfGeom &g, bool split, const double *src, double *host, int64_t ldi,
                            int64_t ldj) {
+    std::lock_guard<std::mutex> lock(turn);
     // the calling thread's device need not be the stream's
     int now = 0;
     hipDevice_t own = 0;

@@ -287,3 +287,22 @@ def test_fields_come_without_pinned_memory(call, dim):
         np.testing.assert_array_equal(wide[:, :p.n + 2, :p.m + 2].reshape(p.full_shape()), a)
         assert (wide[:, p.n + 2:, :] == -7.0).all() and (wide[:, :, p.m + 2:] == -7.0).all()
     """)
+
+
+def test_fields_of_one_context_in_several_threads():
+    run("""
+        os.environ["PF_RESIDENT"] = "0"
+        p, phi = case((33, 21, 13))
+        s = S.Solver(p, phi)
+        values = {"u": 1.0, "v": 2.0, "w": 3.0, "p": 4.0}
+        for f, v in values.items(): s.set_field(f, np.full(p.full_shape(), v))
+        F.fake_hold(1)
+        wrong = []
+        def keep(f):
+            for _ in range(20):
+                if not (s.field(f) == values[f]).all(): wrong.append(f)
+        threads = [threading.Thread(target=keep, args=(f,)) for f in values]
+        for t in threads: t.start()
+        for t in threads: t.join()
+        assert not wrong, wrong
+    """)
