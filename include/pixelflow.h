@@ -134,10 +134,13 @@ int pf_force(pf_ctx *ctx, double *out);
  * needs more).  All calls on one GPU share the array: calls that overlap on one GPU race. */
 int pf_force_noalloc(pf_ctx *ctx, double *out);
 
-/* Device bytes the context holds (admission control sizes cases with this).  A 3D context of
- * a fixed iteration count on up to 4.2 M cells (mixed precision 8.4 M) takes up to 56 (28)
- * bytes more for each cell that is not of porosity 1, or whose neighbours are not, when its
- * porosity is set; without room for them it solves without. */
+/* Device bytes the context holds (admission control sizes cases with this), but for the
+ * coefficients of resident solves (pf_sor_resident): a 3D context of that kind allocates them when
+ * its porosity is set, and solves without where there is no room.  They depend on the porosity:
+ * 3,584 bytes (mixed precision 1,792) for each 64 cells of one colour, a wave's at one height
+ * pair, of which any is not of porosity 1, has a neighbour that is not, or lies at a room's
+ * wall; at most 56 (28) bytes for every cell of the grid, its tiles rounded up to whole waves
+ * and height pairs.  pf_resident_bytes gives what is held. */
 int64_t pf_footprint_bytes(const pf_desc *desc);
 
 /* Wait for all queued work of the context. */
@@ -166,6 +169,8 @@ int pf_sor_fused(const pf_ctx *ctx);
  * launch needs room for all its blocks at once; where other processes' work leaves none it gives
  * up, and the context pauses this form for 16 solves, then for longer, before it tries again. */
 int pf_sor_resident(const pf_ctx *ctx);
+/* Device bytes of the coefficients of resident solves, beside pf_footprint_bytes; 0 if none. */
+int64_t pf_resident_bytes(const pf_ctx *ctx);
 /* 1 if the FP64 colour sweeps read the porosity coded in 4 bytes per value (values FP32
  * holds exactly as floats, the others through a table of at most 2^20 distinct doubles:
  * the same doubles, 4 fewer bytes per cell and sweep; the default past 512 MB of sweep

@@ -1162,6 +1162,8 @@ extern "C" int pf_sor_resident(const pf_ctx *c) {
     return ((c->resident && c->rready) || c->resident2) ? 1 : 0;
 }
 
+extern "C" int64_t pf_resident_bytes(const pf_ctx *c) { return c ? (int64_t)c->rcoef_cap : PF_EINVAL; }
+
 extern "C" int pf_set_timing(pf_ctx *c, int on) {
     if (!c) return PF_EINVAL;
     c->timing = on != 0;

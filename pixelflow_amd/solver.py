@@ -62,7 +62,7 @@ _lib: Optional[ctypes.CDLL] = None
 # Every symbol include/pixelflow.h declares (checked by tests/test_abi.py).
 EXPORTS = ("pf_abi_version", "pf_create", "pf_destroy", "pf_last_error", "pf_set_porosity", "pf_initial",
            "pf_upload", "pf_download", "pf_step", "pf_divergence", "pf_force", "pf_force_noalloc", "pf_footprint_bytes", "pf_sync",
-           "pf_set_timing", "pf_last_sweep_time_us", "pf_sor_kernel", "pf_sor_fused", "pf_sor_resident", "pf_sor_coded", "pf_sor_unit_cells",
+           "pf_set_timing", "pf_last_sweep_time_us", "pf_sor_kernel", "pf_sor_fused", "pf_sor_resident", "pf_resident_bytes", "pf_sor_coded", "pf_sor_unit_cells",
            "pf_probe_copy",
            "pf_batch_create", "pf_batch_destroy", "pf_batch_last_error", "pf_batch_case_bytes", "pf_batch_free_bytes",
            "pf_batch_add", "pf_batch_remove", "pf_batch_count", "pf_batch_step", "pf_batch_download",
@@ -124,6 +124,8 @@ def lib() -> ctypes.CDLL:
     L.pf_sor_kernel.argtypes = [vp]
     L.pf_sor_fused.argtypes = [vp]
     L.pf_sor_resident.argtypes = [vp]
+    L.pf_resident_bytes.restype = ctypes.c_int64
+    L.pf_resident_bytes.argtypes = [vp]
     L.pf_sor_coded.argtypes = [vp]
     L.pf_sor_unit_cells.argtypes = [vp, ctypes.POINTER(ctypes.c_int64)]
     L.pf_probe_copy.argtypes = [ctypes.c_int64, ctypes.c_int, dp]
@@ -274,6 +276,10 @@ class Solver:
     def sor_resident(self) -> bool:
         """True when a fixed count of SOR iterations runs as one launch, the grid on chip."""
         return lib().pf_sor_resident(self._h) == 1
+
+    def resident_bytes(self) -> int:
+        """Device bytes of the coefficients of resident solves, beside footprint_bytes."""
+        return int(lib().pf_resident_bytes(self._h))
 
     def sor_coded(self) -> bool:
         """True when the FP64 sweeps read the porosity coded in 4 bytes per value."""

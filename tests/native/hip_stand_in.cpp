@@ -30,7 +30,7 @@ std::vector<std::string> g_log;
 std::map<size_t, std::deque<std::vector<char>>> g_reads;   // by size: what later device-to-host copies deliver
 // pending: a resident launch not yet waited for
 struct Stream { int pending = 0; unsigned blocks = 0; bool capturing = false; };
-int g_give_up = 0, g_hold_ms = 0;
+int g_give_up = 0, g_good = 0, g_hold_ms = 0;
 unsigned g_blocks = 0, g_most_blocks = 0;
 int g_inflight = 0, g_most = 0;
 size_t g_allocated = 0;
@@ -71,7 +71,7 @@ void fake_reset() {
     g_calls.clear();
     g_log.clear();
     g_reads.clear();
-    g_give_up = g_hold_ms = g_most = 0;
+    g_give_up = g_good = g_hold_ms = g_most = 0;
     g_most_blocks = 0;
     t_last = hipSuccess;
 }
@@ -81,7 +81,9 @@ void fake_fail(const char *fn, int skip, int times, int err) {
     g_faults[fn] = Fault{skip, times, (hipError_t)err};
 }
 // The next `n` resident launches give up.
-void fake_give_up(int n) { g_give_up = n; }
+void fake_give_up(int n) { g_give_up = n; g_good = 0; }
+// The `n` after the next `good` do.
+void fake_give_up_after(int good, int n) { g_good = good; g_give_up = n; }
 // A wait for an event, or for a stream that holds a resident launch, takes this long.
 void fake_hold(int ms) { g_hold_ms = ms; }
 // The next device-to-host copy of `bytes` bytes delivers `data` (a queue per size).
@@ -181,7 +183,10 @@ hipError_t hipMemGetInfo(size_t *f, size_t *t) { *f = *t = (size_t)288 << 30; re
 static hipError_t copy(void *dst, const void *src, size_t n, hipMemcpyKind kind, Stream *s) {
     if (kind == hipMemcpyDeviceToHost && s && s->pending == 1 && n == 8) {
         unsigned long long *count = (unsigned long long *)src;
-        if (g_give_up > 0) {
+        if (g_good > 0) {
+            --g_good;
+            *count += s->blocks;
+        } else if (g_give_up > 0) {
             --g_give_up;
             *count |= GONE;
         } else {

@@ -306,3 +306,41 @@ def test_fields_of_one_context_in_several_threads():
         for t in threads: t.join()
         assert not wrong, wrong
     """)
+
+
+@pytest.mark.parametrize("kind", ["3d", "2d"])
+def test_message_numbers_start_over_on_an_empty_inbox(kind):
+    """Numbers are 32 bits; before they run out the inbox is cleared and they begin again."""
+    run(f"""
+        if {kind!r} == "2d": os.environ["PF_RESIDENT"] = "1,2"
+        p, phi = case((64, 32, 1) if {kind!r} == "2d" else (64, 32, 32), iters=(1 << 28) - 1)
+        used, cleared = 1, 0
+        with S.Solver(p, phi) as s:
+            for step in range(40):
+                a = launches("k_clear_u64")
+                s.step(1)
+                need = p.iter_max if {kind!r} == "2d" else 2 * p.iter_max
+                over = used + need > 0xffffffff
+                used = need + (1 if over else used)
+                cleared += over
+                assert launches("k_clear_u64") - a == 1 + over, step     # the step's own and the inbox
+            assert cleared >= 2 and launches("k_sor_resident") == 40
+    """)
+
+
+def test_a_cycle_that_gives_up_is_swept_alone():
+    """The second of three cycles of a step: one cycle's sweeps and one update each, then a pause."""
+    run("""
+        p, phi = case(iters=60)
+        with S.Solver(p, phi, precision=S.PF_PREC_MIXED, inner_iters=20) as s:
+            F.fake_give_up_after(1, 1)
+            n = launches("k_update")
+            s.step(1)
+            assert launches("k_sor_resident") == 2            # the first, and the one that gave up
+            assert launches("k_sor32") == 2 * 2 * 20           # the second and the third
+            assert launches("k_update") - n == 3
+            for _ in range(5): s.step(1)                        # fifteen more of the pause
+            assert launches("k_sor_resident") == 2
+            s.step(1)
+            assert launches("k_sor_resident") == 5
+    """)
