@@ -29,11 +29,12 @@
 // sor_coefs (FP32: sor32_coefs) built them once per porosity field.
 //
 // Measured, us per half-sweep, one launch per half-sweep / resident: FP64 sphere 256x128x128
-// 17.0 / 9.6, sphere 97x65x49 7.9 / 3.1, room 128^3 13.4 / 8.0; FP32 sphere 256x128x128
-// 10.2 / 6.7.  What bounds it: an exchange takes about 1.6 us however little travels (a
-// 64x64x64 grid on 256 blocks, 1.8 us); a tile of 16384 unit cells takes 5.0 us (FP64: 0.4 us
-// of arithmetic per height pair); a tile around a body, whose waves read seven coefficients a
-// cell, waits about 0.9 us a height pair for them, and its neighbours wait for it.  Tiles of
+// 17.0 / 9.6, sphere 97x65x49 7.9 / 2.8, room 128^3 13.4 / 7.6; FP32 sphere 256x128x128
+// 10.2 / 6.8, room 128^3 8.3 / 4.5.  What bounds it: an exchange takes about 1.6 us however little
+// travels (a 64x64x64 grid on 256 blocks, 1.8 us); a tile of 16384 unit cells takes 5.0 us (FP64:
+// 0.4 us of arithmetic per height pair); a tile around a body, whose waves read seven coefficients
+// a cell, waits about 0.65 us a height pair for them, and its neighbours wait for it; in an FP64
+// room, where nearly all waves read them, all tiles together read 6 to 9 TB/s.  Tiles of
 // 32x32 columns: 64x16, which spread a body over twice the tiles, took 10.6 us on the sphere.
 // Sends at the end of a wave's half-sweep instead of per height pair took 10.4, coefficients
 // fetched a height pair ahead 11.6 (registers spill).
@@ -112,7 +113,9 @@ constexpr int msg_items() { return 4 * 2 * NS * RT + 2 * RMAXT; }
 // Block blockIdx runs on XCD blockIdx % 8.  The tiles of a row of tiles are turned by this
 // much against the row's blocks, so that tiles that are neighbours in y and z, which read
 // coefficients of the same body, are on different XCDs: a body's coefficients then share
-// eight L2s (4 MB each) instead of the one or two that its x range falls on.
+// eight L2s (4 MB each) instead of the one or two that its x range falls on.  us a half-sweep
+// without / with: FP64 boxes 256x128x128 13.1 / 10.2, sphere 10.3 / 9.6, room 128^3 8.2 / 7.6;
+// FP32 8.1 / 7.1, 6.7 / 6.8, 4.8 / 4.5; where bx is no multiple of 8 the same.
 __device__ __forceinline__ int tile_turn(const ResidentPlan &pl, int iy, int iz) {
     return (pl.bx % 8 == 0) ? 2 * iy + 4 * iz : iz;
 }
