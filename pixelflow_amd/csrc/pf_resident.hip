@@ -649,8 +649,9 @@ static double body_tile_us(const ResidentPlan &pl, int elem) {
     const double pairs = (pl.tz + 1) / 2, waves = pl.threads / 64, columns = pl.tx * pl.ty;
     const bool f64 = elem == 8, odd = ((pl.tx | pl.ty) & 1) != 0;
     const double wait = 0.65 * pairs, loads = (f64 ? 0.074 : 0.034) * pairs * waves;
+    const double w2 = wait * wait, l2 = loads * loads;
     const double columns_us = f64 ? (odd ? 2.00e-3 : 1.66e-3) : (odd ? 0.93e-3 : 0.90e-3);
-    return (f64 ? 0.63 : 0.67) + std::pow(std::pow(wait, 4) + std::pow(loads, 4), 0.25) + columns_us * columns +
+    return (f64 ? 0.63 : 0.67) + std::sqrt(std::sqrt(w2 * w2 + l2 * l2)) + columns_us * columns +
            (f64 ? 0.42 : 0.24) * 2 * (pl.tx + pl.ty) * pairs / pl.threads;
 }
 // The same for a tile of unit cells: arithmetic of the fullest SIMD, and the surface.
